@@ -1,11 +1,11 @@
 // Grouped persistent complex GEMM kernels (gfx950 MFMA).
 //
-// Workgroup = 256 threads = 4 wave64s arranged 2x2; a TM x TN output tile
-// per workgroup, each wave owning a (TM/2) x (TN/2) sub-tile made of 16x16
-// MFMA fragments.  K is consumed in chunks of KC (16 or 8) staged through LDS
-// with real and imaginary parts in separate planes (so one MFMA operand is one
-// LDS read); the next chunk is prefetched into registers while the current
-// one is multiplied.  A complex product is four real MFMAs,
+// Workgroup = 4 wave64s arranged 2x2 (8 for the widest FP64 tiles); a TM x TN
+// output tile per workgroup, each wave owning a sub-tile made of 16x16 MFMA
+// fragments.  K is consumed in chunks of KC (16 or 8) staged through LDS
+// as interleaved (re, im) pairs (one LDS read gives both parts of a fragment);
+// the next chunk is prefetched into registers while the current one is
+// multiplied.  A complex product is four real MFMAs,
 //   Cre += Are*Bre + (-Aim)*Bim,   Cim += Are*Bim + Aim*Bre,
 // or three (Gauss): P1 = Are*Bre, P2 = Aim*Bim, P3 = (Are+Aim)*(Bre+Bim),
 //   Cre = P1 - P2,   Cim = P3 - P1 - P2.
@@ -13,7 +13,8 @@
 // MFMA 16x16x4 operand layout (wave64): lane l supplies A[l%16][l/16] and
 // B[l/16][l%16].  Accumulator element v of lane l is D[row][l%16] with
 // row = l/16 + 4v for the f64 instruction and row = 4(l/16) + v for f32
-// (measured on gfx950).
+// (measured on gfx950).  The kernel passes its B as the first operand, so D
+// is the transposed tile: row = column n, l%16 = row m.
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -21,6 +22,7 @@
 #include <map>
 #include <mutex>
 #include <numeric>
+#include <type_traits>
 #include <unordered_map>
 
 #include "gemm.hpp"
@@ -31,7 +33,6 @@ namespace {
 
 constexpr int KCmax = 16;  // largest K chunk staged in LDS
 constexpr int kXcds = 8;   // MI355X accelerator complex dies (one L2 each)
-constexpr int PADL = 4;    // LDS row padding (elements)
 
 // global-address-space access (global_load / global_store rather than
 // flat) through native vector types: HIP's double2/float2 have reference
@@ -97,32 +98,95 @@ template <> struct Mf<float> {
   static __device__ __forceinline__ int row(int fk, int v) { return 4 * fk + v; }
 };
 
+// Raw buffer access: wave-uniform 64-bit base in scalar registers plus a
+// 32-bit per-lane byte offset.  An offset at or past the record limit reads
+// zero without touching memory, which is how elements outside a problem are
+// padded.
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+constexpr uint32_t kBufRecords = 0x7ffffff0u;
+constexpr uint32_t kBufOutside = 0x80000000u;
+constexpr int kBufFlags = 0x00020000;   // raw 32-bit data format
+
+template <typename R> struct BufRaw;
+template <> struct BufRaw<double> {
+  using V = d2v;
+  static __device__ __forceinline__ V load(const char* base, uint32_t records, uint32_t off) {
+    __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, records, kBufFlags);
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  }
+};
+template <> struct BufRaw<float> {
+  using V = f2v;
+  static __device__ __forceinline__ V load(const char* base, uint32_t records, uint32_t off) {
+    __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, records, kBufFlags);
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+  }
+};
+
+// Waves of a workgroup over its tile: 2 x 2, or eight of them for the wide
+// FP64 tiles (a wave's accumulators for more than 32 x 32 FP64 outputs would
+// leave one wave per SIMD).
+template <typename R, int TM, int TN> struct Waves {
+  static constexpr bool kWide = sizeof(R) == 8 && TM * TN > 4096;
+  static constexpr int kM = kWide && TM > TN ? 4 : 2;
+  static constexpr int kN = kWide && TN > TM ? 4 : 2;
+  static constexpr int kThreads = 64 * kM * kN;
+};
+
 // G3: complex products with three real MFMAs (P1 = Ar Br, P2 = Ai Bi,
 // P3 = (Ar + Ai)(Br + Bi); re = P1 - P2, im = P3 - P1 - P2) instead of four;
 // the error stays O(eps |A||B|) per product, as for the four-product form.
 // KC = 8 halves the LDS footprint and the prefetch registers (more resident
-// workgroups where registers allow) at one barrier per 8 instead of 16 k
+// workgroups where registers allow) at one barrier per 8 instead of 16 k.
+//
+// Bound by MFMA issue: a vector instruction of either resident wave stalls the
+// matrix pipe for about three cycles (v_add_f64: six or more; an FP64 MFMA
+// takes 64, an FP32 one 32; an MFMA-only loop reaches 75.8 TFLOP/s in FP64,
+// four 32-bit adds per MFMA 65, eight 56), and two waves per SIMD do not
+// cover a wave's staging, barrier and first LDS reads.  So
+//  - operands come in through buffer loads with a scalar base advanced by
+//    scalar adds and one lane offset per operand; padding is cut off by the
+//    record length;
+//  - LDS holds interleaved (re, im) pairs: a staged element is one store and
+//    a fragment (both parts) one load, without packing or selects;
+//  - staging, cursor and loads stand between the MFMA passes of a chunk's
+//    first k step, the barrier before its last one.
+// About 30 vector instructions per 48 MFMAs are left (16 of them the Gauss
+// sums), from over 200.  Coupled chain, d=64, chi=500: FP64 stages L and R
+// 49.2 / 48.6 -> 39.1 / 39.6 ms (62.5 -> 78.5 TFLOP/s, pipe busy 0.63 -> 0.79),
+// W stages 15.1 / 15.0 -> 12.6 / 12.0 ms (49 GB each: near the copy rate);
+// chi=256 FP32 matvec 12.2 -> 9.4 ms.
 template <typename R, int TM, int TN, bool G3, int KC>
-__global__ __launch_bounds__(256) void grouped_gemm_kernel(const GemmProb* __restrict__ probs,
-                                                           const GemmSeg* __restrict__ segs,
-                                                           const GemmTile* __restrict__ tiles,
-                                                           int ntiles, GemmBases bases) {
+__global__ __launch_bounds__((Waves<R, TM, TN>::kThreads)) void grouped_gemm_kernel(
+    const GemmProb* __restrict__ probs, const GemmSeg* __restrict__ segs, const GemmTile* __restrict__ tiles,
+    int ntiles, GemmBases bases) {
   using C = typename CT<R>::T;
+  using V = typename BufRaw<R>::V;
   using acc_t = typename Mf<R>::acc;
-  constexpr int LDA = TM + PADL;
-  constexpr int LDB = TN + PADL;
-  constexpr int PA = TM * KC / 256;   // A elements per thread per chunk
-  constexpr int PB = TN * KC / 256;   // B elements per thread per chunk
-  constexpr int FM = TM / 32;         // 16-row fragments per wave
-  constexpr int FN = TN / 32;
+  constexpr int ES = sizeof(C);
+  // one element of padding: the rows of a K-contiguous operand, written at
+  // one k per lane, then fall on different banks
+  constexpr int LDA = TM + 1;
+  constexpr int LDB = TN + 1;
+  using WG = Waves<R, TM, TN>;
+  constexpr int NT = WG::kThreads;
+  constexpr int PA = TM * KC / NT;    // A elements per thread per chunk
+  constexpr int PB = TN * KC / NT;    // B elements per thread per chunk
+  constexpr int WTM = TM / WG::kM;    // a wave's sub-tile
+  constexpr int WTN = TN / WG::kN;
+  constexpr int FM = WTM / 16;        // 16-row fragments per wave
+  constexpr int FN = WTN / 16;
+  static_assert(PA * NT == TM * KC && PB * NT == TN * KC, "a chunk divides evenly over the threads");
   // two LDS buffers: chunk c+1 is stored while chunk c is multiplied, so one
   // barrier per chunk suffices
-  __shared__ R sAr[2][KC * LDA], sAi[2][KC * LDA], sBr[2][KC * LDB], sBi[2][KC * LDB];
+  __shared__ alignas(16) V sA[2][KC * LDA];
+  __shared__ alignas(16) V sB[2][KC * LDB];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WG::kM, wn = wave / WG::kM;
   const int fr = lane & 15, fk = lane >> 4;
 
   // XCD-aware order: workgroup b runs on XCD b % 8, so consecutive tiles
@@ -148,265 +212,216 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const GemmProb* __res
         if (G3) accs[G3 ? i : 0][G3 ? j : 0] = acc_t{0, 0, 0, 0};
       }
 
-    // prefetched operands of the next chunk (registers) and their in-bounds flags
-    C ra0[PA], rb0[PB];
-    uint32_t am0 = 0, bm0 = 0;
+    // prefetched operands of one chunk
+    V ra[PA], rb[PB];
     const int send = P.seg0 + P.nseg;
-    // load cursor: segment and k offset of the next chunk to load (plans
-    // hold no empty segments)
-    int cs = P.seg0;
-    int ck = 0;
-    GemmSeg CS;
-    if (cs < send) CS = cload(segs + cs);
+    // layout of the operands (the same for every segment of a problem)
+    const int32_t lay = P.nseg ? cload(segs + P.seg0).flags : 0;
+    const bool akc = lay & kSegAKContig, bnc = lay & kSegBNContig;
 
-    // Address state of the current segment, set up once per segment: the
-    // operand pointers at this tile's batch, first row / column and the
-    // segment's first k, every element's offset from them (32 bits: a tile
-    // spans at most 128 rows or columns and the plans keep strides below
-    // 2^31 / 128), the element stride along k and which elements lie inside
-    // the problem's rows / columns.  A chunk's addresses are then one add per
-    // element (the chunk's k offset is uniform).
-    const C* segA = nullptr;
-    const C* segB = nullptr;
-    int32_t aoff[PA], boff[PB];
-    int64_t sak = 0, sbk = 0;
-    uint32_t arow = 0, bcol = 0;
-    bool akc = false, bnc = false;
-    auto setup = [&](const GemmSeg& G) {
-      const int asp = (G.flags >> 8) & 15, bsp = (G.flags >> 12) & 15;
-      akc = G.flags & kSegAKContig;
-      bnc = G.flags & kSegBNContig;
-      const int32_t csA = static_cast<int32_t>(G.csA), ldB = static_cast<int32_t>(G.ldB);
-      segA = (asp ? reinterpret_cast<const C*>(bases.p[asp]) + reinterpret_cast<intptr_t>(G.A)
-                  : reinterpret_cast<const C*>(G.A)) +
-             static_cast<int64_t>(tl.batch) * G.bsA + (akc ? static_cast<int64_t>(m0) * G.csA : m0);
-      segB = (bsp ? reinterpret_cast<const C*>(bases.p[bsp]) + reinterpret_cast<intptr_t>(G.B)
-                  : reinterpret_cast<const C*>(G.B)) +
-             static_cast<int64_t>(tl.batch) * G.bsB + (bnc ? n0 : static_cast<int64_t>(n0) * G.ldB);
-      sak = akc ? 1 : G.csA;
-      sbk = bnc ? G.ldB : 1;
-      arow = 0;
-      bcol = 0;
-#pragma unroll
-      for (int p = 0; p < PA; ++p) {
-        const int e = tid + p * 256;
-        const int m = akc ? e / KC : e % TM, k = akc ? e % KC : e / TM;
-        aoff[p] = akc ? k + m * csA : m + k * csA;
-        arow |= (m0 + m < M ? 1u : 0u) << p;
+    // Load cursor: segment, k offset in it, its K and its operands.  A wave's
+    // load p covers the 64 consecutive elements 64 wave + kThreads p of the
+    // chunk: M-contiguous A runs over the rows of a k, a K-contiguous operand
+    // over the k of a row.  A lane's byte offset from the load's scalar base
+    // does not depend on p; it spans at most 7 strides (KC = 8, K-contiguous)
+    // of less than 2^24 elements, below 2^31 bytes.  Elements outside the
+    // problem are cut off by the record length: of a K-contiguous operand the
+    // rows past the edge, of an M-contiguous one the k past the segment's end
+    // (its rows past the edge have their lane offset outside).
+    int cs = P.seg0, ck = 0, csK = 0;
+    uint32_t aoff = 0, boff = 0;
+    const char* pa = nullptr;           // this wave's load 0 of the chunk
+    const char* pb = nullptr;
+    int64_t sap = 0, sbp = 0;           // bytes from load p to p + 1
+    int64_t sak = 0, sbk = 0;           // bytes from a chunk to the next
+    uint32_t lda = 0, ldb = 0;          // bytes of a stride
+    const int lk = lane % KC, lr = lane / KC;
+    auto setup = [&]() {
+      const GemmSeg S = cload(segs + cs);
+      csK = S.K;
+      const int asp = (S.flags >> 8) & 15, bsp = (S.flags >> 12) & 15;
+      const C* A = (asp ? reinterpret_cast<const C*>(bases.p[asp]) + reinterpret_cast<intptr_t>(S.A)
+                        : reinterpret_cast<const C*>(S.A)) +
+                   static_cast<int64_t>(tl.batch) * S.bsA;
+      const C* B = (bsp ? reinterpret_cast<const C*>(bases.p[bsp]) + reinterpret_cast<intptr_t>(S.B)
+                        : reinterpret_cast<const C*>(S.B)) +
+                   static_cast<int64_t>(tl.batch) * S.bsB;
+      const int64_t sA = S.csA * ES, sB = S.ldB * ES;
+      lda = static_cast<uint32_t>(sA);
+      ldb = static_cast<uint32_t>(sB);
+      if (akc) {
+        pa = reinterpret_cast<const char*>(A) + (m0 + wave * (64 / KC)) * sA;
+        sap = (NT / KC) * sA;
+        sak = KC * ES;
+        aoff = lr * lda + lk * ES;
+      } else {
+        pa = reinterpret_cast<const char*>(A + m0 + wave * 64 % TM) + (wave * 64 / TM) * sA;
+        sap = (NT / TM) * sA;
+        sak = KC * sA;
+        aoff = m0 + tid % TM < M ? (TM < 64 ? lane % TM * ES + (lane / TM) * lda : lane * ES) : kBufOutside;
       }
-#pragma unroll
-      for (int p = 0; p < PB; ++p) {
-        const int e = tid + p * 256;
-        const int n = bnc ? e % TN : e / KC, k = bnc ? e / TN : e % KC;
-        boff[p] = bnc ? k * ldB + n : k + n * ldB;
-        bcol |= (n0 + n < N ? 1u : 0u) << p;
+      if (bnc) {
+        pb = reinterpret_cast<const char*>(B + n0 + wave * 64 % TN) + (wave * 64 / TN) * sB;
+        sbp = (NT / TN) * sB;
+        sbk = KC * sB;
+        boff = n0 + tid % TN < N ? (TN < 64 ? lane % TN * ES + (lane / TN) * ldb : lane * ES) : kBufOutside;
+      } else {
+        pb = reinterpret_cast<const char*>(B) + (n0 + wave * (64 / KC)) * sB;
+        sbp = (NT / KC) * sB;
+        sbk = KC * ES;
+        boff = lr * ldb + lk * ES;
       }
     };
-    if (cs < send) setup(CS);
+    // steps the cursor to the next chunk; false (and K = 0) past the last one
     auto advance = [&]() {
       ck += KC;
-      if (ck >= CS.K) {
-        ck = 0;
-        ++cs;
-        if (cs < send) {
-          CS = cload(segs + cs);
-          setup(CS);
-        }
-      }
-      return cs < send;
+      pa += sak;
+      pb += sbk;
+      if (ck < csK) return true;
+      ck = 0;
+      csK = 0;
+      if (cs + 1 >= send) return false;
+      ++cs;
+      setup();
+      return true;
     };
-
-    // operand loads of the chunk at k offset kk0 of the current segment:
-    // global address space (not flat, whose completion the LDS waits of the
-    // MFMA loop would also have to wait for) and branch-free: an element
-    // outside the problem reads the segment's first element and is zeroed
-    // when it is staged to LDS, so nothing waits on the loads before the
-    // MFMAs
-    auto load = [&](int kk0, int K, C(&ra)[PA], C(&rb)[PB], uint32_t& amask, uint32_t& bmask) {
-      const int64_t da = static_cast<int64_t>(kk0) * sak, db = static_cast<int64_t>(kk0) * sbk;
-      const int kleft = K - kk0;
+    // K-contiguous operands: rows (columns) of load p inside the problem
+    int arows[PA], bcols[PB];
 #pragma unroll
-      for (int p = 0; p < PA; ++p) {
-        const int e = tid + p * 256;
-        const int k = akc ? e % KC : e / TM;
-        const bool ok = ((arow >> p) & 1u) && k < kleft;
-        // a padding element reads the tile's first element of the segment,
-        // inside the operand's allocation; the empty asm keeps the compiler
-        // from turning the select into two loads under divergent branches
-        int64_t o = ok ? aoff[p] + da : 0;
-        asm("" : "+v"(o));
-        ra[p] = gload(segA + o);
-        amask = ok ? (amask | (1u << p)) : (amask & ~(1u << p));
-      }
+    for (int p = 0; p < PA; ++p)
+      arows[p] = __builtin_amdgcn_readfirstlane(min(max(M - m0 - (wave * 64 + p * NT) / KC, 0), 64 / KC));
 #pragma unroll
-      for (int p = 0; p < PB; ++p) {
-        const int e = tid + p * 256;
-        const int k = bnc ? e / TN : e % KC;
-        const bool ok = ((bcol >> p) & 1u) && k < kleft;
-        int64_t o = ok ? boff[p] + db : 0;
-        asm("" : "+v"(o));
-        rb[p] = gload(segB + o);
-        bmask = ok ? (bmask | (1u << p)) : (bmask & ~(1u << p));
-      }
+    for (int p = 0; p < PB; ++p)
+      bcols[p] = __builtin_amdgcn_readfirstlane(min(max(N - n0 - (wave * 64 + p * NT) / KC, 0), 64 / KC));
+    // record length of load p of an operand with T rows (columns) a chunk,
+    // `in` of the load's inside the problem, at stride ld
+    auto records = [&](bool kc, int T, int in, uint32_t ld, int p, int kleft) -> uint32_t {
+      const int k = (wave * 64 + p * NT) / T;
+      const uint32_t rk = kleft > 0 ? in * ld : 0;
+      const uint32_t rm = k < kleft ? (T < 64 && k + 1 >= kleft ? ld : kBufRecords) : 0;
+      return __builtin_amdgcn_readfirstlane(kc ? rk : rm);
     };
-    auto store = [&](const GemmSeg& G, int buf, const C(&ra)[PA], const C(&rb)[PB], uint32_t amask,
-                     uint32_t bmask) {
-      R* __restrict__ pAr = sAr[buf];
-      R* __restrict__ pAi = sAi[buf];
-      R* __restrict__ pBr = sBr[buf];
-      R* __restrict__ pBi = sBi[buf];
-      const bool cA = G.flags & kSegConjA, cB = G.flags & kSegConjB, al = G.flags & kSegAlpha;
-      const R are = static_cast<R>(G.alpha_re), aim = static_cast<R>(G.alpha_im);
-      const bool akc = G.flags & kSegAKContig;
+    // loads of the chunk at the cursor (past the last one: nothing)
+    auto load = [&]() {
+      const int kleft = csK - ck;
+      const uint32_t ao = akc && lk >= kleft ? kBufOutside : aoff;
+      const uint32_t bo = !bnc && lk >= kleft ? kBufOutside : boff;
 #pragma unroll
-      for (int p = 0; p < PA; ++p) {
-        const int e = tid + p * 256;
-        const int m = akc ? e / KC : e % TM, k = akc ? e % KC : e / TM;
-        const bool ok = (amask >> p) & 1u;
-        R xr = ok ? ra[p].x : R(0), xi = ok ? (cA ? -ra[p].y : ra[p].y) : R(0);
-        if (al) {
-          const R tr = xr * are - xi * aim;
-          xi = xr * aim + xi * are;
-          xr = tr;
-        }
-        pAr[k * LDA + m] = xr;
-        pAi[k * LDA + m] = xi;
-      }
-      if (G.flags & kSegBNContig) {
+      for (int p = 0; p < PA; ++p)
+        ra[p] = BufRaw<R>::load(pa + p * sap, records(akc, TM, arows[p], lda, p, kleft), ao);
 #pragma unroll
-        for (int p = 0; p < PB; ++p) {
-          const int e = tid + p * 256;
-          const int n = e % TN, k = e / TN;
-          const bool ok = (bmask >> p) & 1u;
-          pBr[k * LDB + n] = ok ? rb[p].x : R(0);
-          pBi[k * LDB + n] = ok ? (cB ? -rb[p].y : rb[p].y) : R(0);
-        }
+      for (int p = 0; p < PB; ++p)
+        rb[p] = BufRaw<R>::load(pb + p * sbp, records(!bnc, TN, bcols[p], ldb, p, kleft), bo);
+    };
+    // stages the loaded chunk, conjugated where the problem asks for it (H_eff
+    // problems do not)
+    auto stage = [&](int buf, auto conj) {
+      const bool cA = decltype(conj)::value && (lay & kSegConjA), cB = decltype(conj)::value && (lay & kSegConjB);
+      V* __restrict__ dA = sA[buf];
+      V* __restrict__ dB = sB[buf];
+      if (akc) {
+#pragma unroll
+        for (int p = 0; p < PA; ++p)
+          dA[(tid % KC) * LDA + tid / KC + p * (NT / KC)] = V{ra[p].x, cA ? -ra[p].y : ra[p].y};
       } else {
 #pragma unroll
-        for (int p = 0; p < PB; ++p) {
-          const int e = tid + p * 256;
-          const int k = e % KC, n = e / KC;
-          const bool ok = (bmask >> p) & 1u;
-          pBr[k * LDB + n] = ok ? rb[p].x : R(0);
-          pBi[k * LDB + n] = ok ? (cB ? -rb[p].y : rb[p].y) : R(0);
+        for (int p = 0; p < PA; ++p)
+          dA[(tid / TM + p * (NT / TM)) * LDA + tid % TM] = V{ra[p].x, cA ? -ra[p].y : ra[p].y};
+      }
+      if (bnc) {
+#pragma unroll
+        for (int p = 0; p < PB; ++p)
+          dB[(tid / TN + p * (NT / TN)) * LDB + tid % TN] = V{rb[p].x, cB ? -rb[p].y : rb[p].y};
+      } else {
+#pragma unroll
+        for (int p = 0; p < PB; ++p)
+          dB[(tid % KC) * LDB + tid / KC + p * (NT / KC)] = V{rb[p].x, cB ? -rb[p].y : rb[p].y};
+      }
+    };
+    auto store = [&](int buf) {
+      if (lay & (kSegConjA | kSegConjB)) stage(buf, std::true_type{});
+      else stage(buf, std::false_type{});
+    };
+
+    // fragments of one k step (four k), double buffered in registers
+    V fa[2][FM], fb[2][FN];
+    auto frag = [&](int buf, int ks, int slot) {
+      const int kr = ks * 4 + fk;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[slot][i] = sA[buf][kr * LDA + wm * WTM + fr + i * 16];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) fb[slot][j] = sB[buf][kr * LDB + wn * WTN + fr + j * 16];
+    };
+    // One pass of a k step's MFMAs over the fragments, FM*FN of them on
+    // different accumulators (three passes with G3, else four).  B is the
+    // instruction's first operand: the accumulator's lanes then run along m,
+    // and a store instruction writes 16 consecutive rows.
+    auto pass = [&](int slot, int w) {
+      R sb[FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) sb[j] = fb[slot][j].x + fb[slot][j].y;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const V a = fa[slot][i];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const V b = fb[slot][j];
+          if constexpr (G3) {
+            if (w == 0) accr[i][j] = Mf<R>::mma(b.x, a.x, accr[i][j]);
+            if (w == 1) acci[i][j] = Mf<R>::mma(b.y, a.y, acci[i][j]);
+            if (w == 2) accs[i][j] = Mf<R>::mma(sb[j], a.x + a.y, accs[i][j]);
+          } else {
+            if (w == 0) accr[i][j] = Mf<R>::mma(b.x, a.x, accr[i][j]);
+            if (w == 1) acci[i][j] = Mf<R>::mma(b.y, a.x, acci[i][j]);
+            if (w == 2) accr[i][j] = Mf<R>::mma(b.y, -a.y, accr[i][j]);
+            if (w == 3) acci[i][j] = Mf<R>::mma(b.x, a.y, acci[i][j]);
+          }
         }
       }
     };
-
-    auto compute = [&](int buf) {
-      const R* __restrict__ cAr = sAr[buf];
-      const R* __restrict__ cAi = sAi[buf];
-      const R* __restrict__ cBr = sBr[buf];
-      const R* __restrict__ cBi = sBi[buf];
-      // fragments of step ks+1 are read from LDS before the MFMAs of step ks
-      // are issued, so their latency hides behind those MFMAs (tiles up to
-      // 64x64; the 128-wide tiles have no registers to spare and read each
-      // step's fragments just before its MFMAs)
-      constexpr bool kPipe = TM * TN <= 4096;
-      R far_[2][FM], fai_[2][FM], fbr_[2][FN], fbi_[2][FN];
-      auto frag = [&](int ks, int slot) {
-        const int kr = ks * 4 + fk;
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          far_[slot][i] = cAr[kr * LDA + wm * (TM / 2) + i * 16 + fr];
-          fai_[slot][i] = cAi[kr * LDA + wm * (TM / 2) + i * 16 + fr];
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          fbr_[slot][j] = cBr[kr * LDB + wn * (TN / 2) + j * 16 + fr];
-          fbi_[slot][j] = cBi[kr * LDB + wn * (TN / 2) + j * 16 + fr];
-        }
-      };
-      if (kPipe) frag(0, 0);
-#pragma unroll
-      for (int ks = 0; ks < KC / 4; ++ks) {
-        const int cur = kPipe ? (ks & 1) : 0;
-        if (!kPipe) frag(ks, 0);
-        else if (ks + 1 < KC / 4) frag(ks + 1, cur ^ 1);
-        R ar[FM], ai[FM], br[FN], bi[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          ar[i] = far_[cur][i];
-          ai[i] = fai_[cur][i];
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          br[j] = fbr_[cur][j];
-          bi[j] = fbi_[cur][j];
-        }
-        if constexpr (G3) {
-          // three passes; an accumulator is revisited FM*FN MFMAs later
-          R sa[FM], sb[FN];
-#pragma unroll
-          for (int i = 0; i < FM; ++i) sa[i] = ar[i] + ai[i];
-#pragma unroll
-          for (int j = 0; j < FN; ++j) sb[j] = br[j] + bi[j];
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) accr[i][j] = Mf<R>::mma(ar[i], br[j], accr[i][j]);
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acci[i][j] = Mf<R>::mma(ai[i], bi[j], acci[i][j]);
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) accs[i][j] = Mf<R>::mma(sa[i], sb[j], accs[i][j]);
-        } else {
-          // four passes over the fragments so that consecutive MFMAs never
-          // depend on each other (each accumulator is revisited 2*FM*FN
-          // instructions later)
-          R nai[FM];
-#pragma unroll
-          for (int i = 0; i < FM; ++i) nai[i] = -ai[i];
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) accr[i][j] = Mf<R>::mma(ar[i], br[j], accr[i][j]);
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acci[i][j] = Mf<R>::mma(ar[i], bi[j], acci[i][j]);
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) accr[i][j] = Mf<R>::mma(nai[i], bi[j], accr[i][j]);
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acci[i][j] = Mf<R>::mma(ai[i], br[j], acci[i][j]);
-        }
-      }
-    };
-
-    int buf = 0;
+    constexpr int kPasses = G3 ? 3 : 4;
+    constexpr int KS = KC / 4;
     if (cs < send) {
-      GemmSeg S0 = CS;
-      load(ck, S0.K, ra0, rb0, am0, bm0);
-      store(S0, 0, ra0, rb0, am0, bm0);
+      setup();
+      load();
+      store(0);
+      bool more = advance();            // whether the registers hold a chunk
+      load();
       __syncthreads();
-      // chunk c+1 is loaded into registers while chunk c is multiplied from
-      // LDS, then staged into the other LDS buffer.  The load is issued
-      // unconditionally (past the last chunk it re-reads the last segment and
-      // is never staged), so every path has the same loads in flight.
-      for (;;) {
-        const bool v1 = advance();
-        const GemmSeg S1 = CS;
-        load(ck, S1.K, ra0, rb0, am0, bm0);
-        // keep every load of the next chunk ahead of the MFMAs (the scheduler
-        // would otherwise sink some of them next to their LDS stores, where
-        // their whole latency is exposed)
-        __builtin_amdgcn_sched_barrier(0);
-        compute(buf);
-        // the other LDS buffer was last read before the previous barrier
-        if (v1) store(S1, buf ^ 1, ra0, rb0, am0, bm0);
-        __syncthreads();
-        buf ^= 1;
-        if (!v1) break;
+      frag(0, 0, 0);
+      // While chunk c is multiplied, chunk c + 1 (in the registers) is staged
+      // into the other LDS buffer and chunk c + 2 loaded; both stand between
+      // MFMA passes.  The barrier stands before the last k step, whose
+      // fragments are in registers by then, and the next chunk's first
+      // fragments are read ahead of that step's MFMAs, so that neither wait
+      // leaves the pipe idle.  Nothing here is conditional: past the last
+      // chunk the loads read nothing, and what they stage is not used.
+      for (int buf = 0;; buf ^= 1) {
+        bool next = false;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int cur = ks & 1;
+          if (ks + 1 < KS) {
+            frag(buf, ks + 1, cur ^ 1);
+          } else {
+            // (the scheduler would move the step's MFMAs ahead of the barrier)
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            frag(buf ^ 1, 0, cur ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          pass(cur, 0);
+          // the other LDS buffer was last read before the previous barrier
+          if (ks == 0) store(buf ^ 1);
+          pass(cur, 1);
+          if (ks == 0) next = advance();
+          pass(cur, 2);
+          if (ks == 0) load();
+          if (kPasses == 4) pass(cur, 3);
+        }
+        if (!more) break;
+        more = next;
       }
-    } else {
-      __syncthreads();
     }
 
     // epilogue
@@ -415,16 +430,16 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const GemmProb* __res
                       : reinterpret_cast<C*>(P.C)) +
             static_cast<int64_t>(tl.batch) * P.bsC;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int n = n0 + wn * (TN / 2) + j * 16 + fr;
+      for (int v = 0; v < 4; ++v) {
+        const int n = n0 + wn * WTN + j * 16 + Mf<R>::row(fk, v);
         if (n >= N) continue;
+        C* col = Cp + static_cast<int64_t>(n) * P.csC;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = m0 + wm * (TM / 2) + i * 16 + Mf<R>::row(fk, v);
+        for (int i = 0; i < FM; ++i) {
+          const int m = m0 + wm * WTM + i * 16 + fr;
           if (m < M) {
-            C* dst = Cp + m + static_cast<int64_t>(n) * P.csC;
             C val;
             if constexpr (G3) {
               const R p1 = accr[i][j][v], p2 = acci[i][j][v];
@@ -435,14 +450,15 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const GemmProb* __res
               val.y = acci[i][j][v];
             }
             if (P.beta) {
-              const C old = gload(dst);
+              const C old = gload(col + m);
               val.x += old.x;
               val.y += old.y;
             }
-            gstore(dst, val);
+            gstore(col + m, val);
           }
         }
       }
+    // the next tile's first chunk overwrites an LDS buffer of this one
     __syncthreads();
   }
 }
@@ -467,7 +483,6 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmProb* __rest
   __shared__ const C* sStepA[kSkinnySteps];    // A column of the step, batch and k applied
   __shared__ int sStepB[kSkinnySteps];         // first element of its B row in sBr / sBi
   __shared__ int sStepF[kSkinnySteps];         // segment flags
-  __shared__ R sStepAr[kSkinnySteps], sStepAi[kSkinnySteps];
   __shared__ int sSegK[kSkinnySegs], sSegOff[kSkinnySegs], sSegStep[kSkinnySegs];
   const int tid = threadIdx.x;
   // XCD-aware order, as for the tiles: consecutive items (the problems of
@@ -516,8 +531,6 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmProb* __rest
         sStepA[st + tid] = Ab + static_cast<int64_t>(tid) * G.csA;
         sStepB[st + tid] = off + tid * N;
         sStepF[st + tid] = G.flags;
-        sStepAr[st + tid] = static_cast<R>(G.alpha_re);
-        sStepAi[st + tid] = static_cast<R>(G.alpha_im);
       }
     }
     __syncthreads();
@@ -534,13 +547,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmProb* __rest
       for (int u = 0; u < 8; ++u) {
         if (j0 + u >= nsteps) break;
         const int j = j0 + u, fl = sStepF[j], bo = sStepB[j];
-        R xr = a[u].x, xi = (fl & kSegConjA) ? -a[u].y : a[u].y;
-        if (fl & kSegAlpha) {
-          const R are = sStepAr[j], aim = sStepAi[j];
-          const R tr = xr * are - xi * aim;
-          xi = xr * aim + xi * are;
-          xr = tr;
-        }
+        const R xr = a[u].x, xi = (fl & kSegConjA) ? -a[u].y : a[u].y;
 #pragma unroll
         for (int n = 0; n < kSkinnyN; ++n) {
           if (n >= N) break;
@@ -594,14 +601,14 @@ void launch_shape(const GemmPlan& plan, const LaunchCfg& c, int shape, hipStream
   const GemmTile* tiles = plan.d_tiles[c.tile_mode][shape].get();
   const GemmProb* P = plan.d_probs.get();
   const GemmSeg* S = plan.d_segs.get();
-  if (c.algo == kAlgo3M && c.kc == 8)
-    hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, true, 8>), dim3(grid), dim3(256), 0, s, P, S, tiles, nt, bases);
-  else if (c.algo == kAlgo3M)
-    hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, true, 16>), dim3(grid), dim3(256), 0, s, P, S, tiles, nt, bases);
-  else if (c.kc == 8)
-    hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, false, 8>), dim3(grid), dim3(256), 0, s, P, S, tiles, nt, bases);
-  else
-    hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, false, 16>), dim3(grid), dim3(256), 0, s, P, S, tiles, nt, bases);
+  auto go = [&](auto g3, auto kc) {
+    hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, decltype(g3)::value, decltype(kc)::value>), dim3(grid),
+                       dim3(Waves<R, TM, TN>::kThreads), 0, s, P, S, tiles, nt, bases);
+  };
+  using K8 = std::integral_constant<int, 8>;
+  using K16 = std::integral_constant<int, 16>;
+  if (c.algo == kAlgo3M) c.kc == 8 ? go(std::true_type{}, K8{}) : go(std::true_type{}, K16{});
+  else c.kc == 8 ? go(std::false_type{}, K8{}) : go(std::false_type{}, K16{});
   HIP_CHECK(hipGetLastError());
 }
 
@@ -643,17 +650,19 @@ void GemmPlan::set_group(int prob, int64_t g) {
 }
 
 void GemmPlan::add_segment(int prob, const void* A, int64_t csA, int64_t bsA, const void* B,
-                           int64_t ldB, int64_t bsB, int K, int flags, double are, double aim) {
+                           int64_t ldB, int64_t bsB, int K, int flags) {
   if (K <= 0) return;   // contributes nothing; the kernels assume K >= 1
   GemmProb& p = probs[prob];
   CAM_REQUIRE(p.seg0 + p.nseg == static_cast<int32_t>(segs.size()),
               "segments of a problem must be added contiguously");
-  // the kernels address an element of a tile by a 32-bit offset from the
-  // tile's first element: at most 128 rows / columns (and KC <= 16 k) times
-  // the stride must stay below 2^31
-  constexpr int64_t kOffLimit = (int64_t(1) << 31) - 256;
-  CAM_REQUIRE(csA >= 0 && ldB >= 0 && csA * 128 < kOffLimit && ldB * 128 < kOffLimit,
+  // the kernels address an element of a load by a 32-bit byte offset (at most
+  // seven strides of 16-byte elements) and cut padding off by record lengths
+  // that count whole strides
+  constexpr int64_t kStrideLimit = (int64_t(1) << 24) - 2;
+  CAM_REQUIRE(csA >= 0 && ldB >= 0 && csA <= kStrideLimit && ldB <= kStrideLimit,
               "add_segment: operand stride too large for 32-bit tile offsets");
+  CAM_REQUIRE(csA >= ((flags & kSegAKContig) ? K : p.M) && ldB >= ((flags & kSegBNContig) ? p.N : K),
+              "add_segment: operand stride below the contiguous extent");
   GemmSeg g{};
   g.A = A;
   g.B = B;
@@ -663,9 +672,9 @@ void GemmPlan::add_segment(int prob, const void* A, int64_t csA, int64_t bsA, co
   g.bsB = bsB;
   g.K = K;
   g.flags = flags;
-  g.alpha_re = are;
-  g.alpha_im = aim;
-  if (are != 1.0 || aim != 0.0) g.flags |= kSegAlpha;
+  // the kernels read layout and conjugation once per problem
+  CAM_REQUIRE(p.nseg == 0 || ((segs[p.seg0].flags ^ g.flags) & 0xff) == 0,
+              "segments of a problem must share their layout and conjugation flags");
   segs.push_back(g);
   p.nseg++;
   flops += 8.0 * double(p.M) * double(p.N) * double(K) * double(p.batch);

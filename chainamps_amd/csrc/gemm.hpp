@@ -1,7 +1,7 @@
 // Grouped, persistent complex GEMM over uneven QN blocks.
 //
 // One launch covers a list of problems.  Problem p computes
-//   C_p[m,n] (+)= sum_s alpha_s * op(A_s)[m,k] * op(B_s)[k,n]
+//   C_p[m,n] (+)= sum_s op(A_s)[m,k] * op(B_s)[k,n]
 // over its K-segments s (every QN-compatible block pair contributing to the
 // same output block), optionally batched (strided) -- the sum over
 // segments is accumulated in registers, so every output tile is written
@@ -28,7 +28,6 @@ enum : int32_t {
   kSegConjA = 1,
   kSegConjB = 2,
   kSegBNContig = 4,   // B(k,n) at k*rsB + n   (else k + n*csB)
-  kSegAlpha = 8,      // multiply A by alpha
   kSegAKContig = 32,  // A(m,k) at k + m*csA   (else m + k*csA)
 };
 
@@ -50,7 +49,6 @@ struct GemmSeg {
   int64_t bsA, bsB;   // batch strides (elements)
   int32_t K;
   int32_t flags;
-  double alpha_re, alpha_im;
 };
 
 struct GemmProb {
@@ -130,7 +128,7 @@ struct GemmPlan {
   int add_problem(void* C, int64_t csC, int M, int N, int batch, int64_t bsC, int beta,
                   int cspace = 0);
   void add_segment(int prob, const void* A, int64_t csA, int64_t bsA, const void* B, int64_t ldB,
-                   int64_t bsB, int K, int flags, double are = 1.0, double aim = 0.0);
+                   int64_t bsB, int K, int flags);
   void set_group(int prob, int64_t g);
   // tile-shape policy for both precisions (see LaunchCfg::tile_mode)
   void choose_tiles(int mode);
