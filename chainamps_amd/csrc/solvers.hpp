@@ -52,6 +52,22 @@ void hermitian_eig(Ctx& ctx, cplx* A, int64_t n, double* w);
 void jordan_wielandt_svd(Ctx& ctx, const cplx* B, int64_t ldb, int64_t m, int64_t n, int64_t k,
                          std::vector<double>& S, cplx* U, cplx* Vh);
 
+// Full decompositions of dense blocks by one-sided Jacobi, all of a call
+// together: A (m x n, column-major, not changed), weight = |A|_F^2, U (m x k)
+// and Vh (k x n) or null for the values only, k = min(m, n).  The result
+// tells which blocks were decomposed (one that did not converge is not).
+struct JacobiItem {
+  const cplx* A;
+  int64_t m, n;
+  double weight;
+  cplx* U;
+  cplx* Vh;
+  std::vector<double>* S;
+};
+constexpr int64_t kJacobiMaxCols = 1024;
+bool jacobi_svd_fits(int64_t m, int64_t n);
+std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items);
+
 // MPX_matrix::SVD with the reference truncation rule.
 void svd_truncate(Ctx& ctx, const BSTensor& theta, int64_t D, double max_trunc, TensorPtr& U,
                   TensorPtr& Vd, std::vector<double>& values, double& discarded);

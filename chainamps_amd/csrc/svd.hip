@@ -9,7 +9,8 @@
 //   * the dense block keeps only non-empty rows and columns
 //     (TranslationBlock, sparse_interface.hpp:353-371) and is decomposed
 //     by economy SVD (the reference calls zgesdd with JOB='S',
-//     dense_matrix_functions.cpp:276-337; here rocSOLVER zgesvd);
+//     dense_matrix_functions.cpp:276-337; here jacobi.hip up to 1024 columns
+//     and 1200 rows, rocSOLVER zgesvd beyond and where that does not converge);
 //   * all singular values are sorted descending (ties: block order, then
 //     index inside the block -- std::sort leaves ties unspecified), the
 //     kept length is min(D, #values) (D=0: all), cut further while the
@@ -117,6 +118,25 @@ __global__ void gather2d_kernel(const GatherJob* jobs, int njobs) {
   }
 }
 
+// per-workgroup partial sums of squared moduli: out[job][workgroup]
+struct WeightJob {
+  const double2* p;
+  int64_t n;
+};
+__global__ __launch_bounds__(256) void weight_kernel(const WeightJob* __restrict__ jobs, double* __restrict__ out) {
+  __shared__ double part[4];
+  const WeightJob J = jobs[blockIdx.y];
+  double w = 0.0;
+  for (int64_t e = blockIdx.x * int64_t(256) + threadIdx.x; e < J.n; e += int64_t(gridDim.x) * 256) {
+    const double2 v = J.p[e];
+    w += v.x * v.x + v.y * v.y;
+  }
+  for (int o = 32; o > 0; o >>= 1) w += __shfl_down(w, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.y * int64_t(gridDim.x) + blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 template <typename J, typename K>
 void run_jobs(K kernel, const std::vector<J>& jobs, hipStream_t s) {
   if (jobs.empty()) return;
@@ -148,7 +168,9 @@ struct Group {
   int64_t first_col = 0;                         // GetAllBlockColumns order key
   double weight = 0.0;
   int64_t k = 0;                                 // number of singular values
-  DevBuf<cplx> A, U, Vh;
+  cplx* A = nullptr;                             // dense compact matrix (in the call's buffer)
+  DevBuf<cplx> U, Vh;                            // the block's own vectors, if not in a shared buffer
+  cplx *Up = nullptr, *Vp = nullptr;             // U (mg x k), V^dagger (k x ng)
   std::vector<double> S;
   bool truncated = false;                        // only the leading k values computed
   double tail = 0.0;                             // weight - sum S^2 when truncated
@@ -257,7 +279,6 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
   }
 
   // ---- assemble dense group matrices and decompose -----------------------
-  DevBuf<cplx> partial(static_cast<size_t>(multi_dot_blocks(int64_t(1) << 40))), dcoef(64);   // k = 1 below
   const char* ev = std::getenv("CAM_SVD_EXACT");
   const bool exact_only = ev && *ev && *ev != '0';
   // CAM_SVD_TRACE=1 prints the path and time of every decomposed block
@@ -281,12 +302,14 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     // values only: no singular vectors (U, V^dagger are 1-element placeholders)
     g.U.alloc(values_only ? 1 : g.mg * g.k);
     g.Vh.alloc(values_only ? 1 : g.k * g.ng);
+    g.Up = g.U.get();
+    g.Vp = g.Vh.get();
     lb.dS.ensure(g.k);
     lb.dE.ensure(std::max<int64_t>(g.k, 1));
     const rocblas_svect sv = values_only ? rocblas_svect_none : rocblas_svect_singular;
     const rocblas_status st = rocsolver_zgesvd(
         static_cast<rocblas_handle>(lane.blas_handle()), sv, sv, static_cast<rocblas_int>(g.mg),
-        static_cast<rocblas_int>(g.ng), reinterpret_cast<rocblas_double_complex*>(g.A.get()),
+        static_cast<rocblas_int>(g.ng), reinterpret_cast<rocblas_double_complex*>(g.A),
         static_cast<rocblas_int>(g.mg), lb.dS.get(), reinterpret_cast<rocblas_double_complex*>(g.U.get()),
         static_cast<rocblas_int>(values_only ? 1 : g.mg), reinterpret_cast<rocblas_double_complex*>(g.Vh.get()),
         static_cast<rocblas_int>(values_only ? 1 : g.k), lb.dE.get(), rocblas_outofplace, lb.dinfo.get());
@@ -297,7 +320,6 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     HIP_CHECK(hipMemcpyAsync(&info, lb.dinfo.get(), sizeof(int), hipMemcpyDeviceToHost, ls));
     HIP_CHECK(hipStreamSynchronize(ls));
     CAM_REQUIRE(info == 0, "blockwise SVD did not converge");
-    g.A.reset();
   };
   auto timed_full_svd = [&](Ctx& lane, LaneBufs& lb, Group& g) {
     const auto t1 = std::chrono::steady_clock::now();
@@ -317,58 +339,91 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     bool full;
   };
   std::vector<Pending> pending;
-  for (size_t gi = 0; gi < glist.size(); ++gi) {
-    Group& g = *glist[gi];
-    if (g.mg == 0 || g.ng == 0) continue;
-    CAM_REQUIRE(g.mg < (int64_t(1) << 31) && g.ng < (int64_t(1) << 31), "SVD block too large");
-    g.A.alloc(g.mg * g.ng);
-    launch_zero(g.A.get(), g.mg * g.ng * sizeof(cplx), s);
-    // scatter the blocks: gather2d with the output as the compact matrix
+  // every group's compact dense matrix, gathered in one launch into one buffer
+  int64_t atot = 0, amax = 0;
+  for (Group* g : glist) {
+    if (g->mg == 0 || g->ng == 0) continue;
+    CAM_REQUIRE(g->mg < (int64_t(1) << 31) && g->ng < (int64_t(1) << 31), "SVD block too large");
+    atot += g->mg * g->ng;
+    amax = std::max(amax, g->mg * g->ng);
+  }
+  DevBuf<cplx> abuf(static_cast<size_t>(std::max<int64_t>(atot, 1)));
+  launch_zero(abuf.get(), atot * static_cast<int64_t>(sizeof(cplx)), s);
+  {
     std::vector<GatherJob> jobs;
-    std::vector<std::vector<int64_t>> keep;
-    for (int b : g.blocks) {
-      const Block& bl = th.blocks[b];
-      std::vector<int32_t> rs(bl.sec.begin(), bl.sec.begin() + r), cs(bl.sec.begin() + r, bl.sec.end());
-      const int ri = g.rpos[rs], ci = g.cpos[cs];
-      // iterate over compact rows/cols that this block covers
-      std::vector<int64_t> rr, cc, orow, ocol;
-      for (int64_t i = 0; i < g.rows[ri].size; ++i)
-        if (g.rmap[g.roff[ri] + i] >= 0) { rr.push_back(i); orow.push_back(g.rmap[g.roff[ri] + i]); }
-      for (int64_t j = 0; j < g.cols[ci].size; ++j)
-        if (g.cmap[g.coff[ci] + j] >= 0) { cc.push_back(j); ocol.push_back(g.cmap[g.coff[ci] + j]); }
-      if (rr.empty() || cc.empty()) continue;
-      // compact rows/cols of one block are contiguous ranges in the group
-      // matrix (tuples are laid out back to back): out = A + orow0 + ocol0*mg
-      keep.push_back(rr);
-      keep.push_back(cc);
-      GatherJob j{};
-      j.in = reinterpret_cast<const double2*>(th.data.get() + bl.offset);
-      j.out = reinterpret_cast<double2*>(g.A.get() + orow.front() + ocol.front() * g.mg);
-      j.M = static_cast<int64_t>(rr.size());
-      j.N = static_cast<int64_t>(cc.size());
-      j.ldo = g.mg;
-      j.rs = 1;
-      j.cs = g.rows[ri].size;
-      j.thr = 0.0;
-      jobs.push_back(j);
-    }
-    // upload the row/col maps
+    std::vector<WeightJob> wjobs;
+    std::vector<Group*> wgroups;
     std::vector<int64_t> flat;
-    std::vector<size_t> at;
-    for (auto& v : keep) { at.push_back(flat.size()); flat.insert(flat.end(), v.begin(), v.end()); }
+    std::vector<std::pair<size_t, size_t>> at;
+    int64_t off = 0;
+    for (Group* gp : glist) {
+      Group& g = *gp;
+      if (g.mg == 0 || g.ng == 0) continue;
+      g.A = abuf.get() + off;
+      off += g.mg * g.ng;
+      wjobs.push_back(WeightJob{reinterpret_cast<const double2*>(g.A), g.mg * g.ng});
+      wgroups.push_back(gp);
+      for (int b : g.blocks) {
+        const Block& bl = th.blocks[b];
+        std::vector<int32_t> rs(bl.sec.begin(), bl.sec.begin() + r), cs(bl.sec.begin() + r, bl.sec.end());
+        const int ri = g.rpos[rs], ci = g.cpos[cs];
+        // compact rows/cols of one block are contiguous ranges in the group
+        // matrix (tuples are laid out back to back): out = A + orow0 + ocol0*mg
+        const size_t a0 = flat.size();
+        int64_t orow = -1, ocol = -1;
+        for (int64_t i = 0; i < g.rows[ri].size; ++i)
+          if (g.rmap[g.roff[ri] + i] >= 0) {
+            if (orow < 0) orow = g.rmap[g.roff[ri] + i];
+            flat.push_back(i);
+          }
+        const size_t c0 = flat.size();
+        for (int64_t j = 0; j < g.cols[ci].size; ++j)
+          if (g.cmap[g.coff[ci] + j] >= 0) {
+            if (ocol < 0) ocol = g.cmap[g.coff[ci] + j];
+            flat.push_back(j);
+          }
+        if (orow < 0 || ocol < 0) {
+          flat.resize(a0);
+          continue;
+        }
+        at.push_back({a0, c0});
+        GatherJob j{};
+        j.in = reinterpret_cast<const double2*>(th.data.get() + bl.offset);
+        j.out = reinterpret_cast<double2*>(g.A + orow + ocol * g.mg);
+        j.M = static_cast<int64_t>(c0 - a0);
+        j.N = static_cast<int64_t>(flat.size() - c0);
+        j.ldo = g.mg;
+        j.rs = 1;
+        j.cs = g.rows[ri].size;
+        j.thr = 0.0;
+        jobs.push_back(j);
+      }
+    }
     DevBuf<int64_t> dmaps(std::max<size_t>(flat.size(), 1));
     dmaps.upload(flat.data(), flat.size(), s);
     for (size_t q = 0; q < jobs.size(); ++q) {
-      jobs[q].r = dmaps.get() + at[2 * q];
-      jobs[q].c = dmaps.get() + at[2 * q + 1];
+      jobs[q].r = dmaps.get() + at[q].first;
+      jobs[q].c = dmaps.get() + at[q].second;
     }
     run_jobs(gather2d_kernel, jobs, s);
-    // group weight (sum of squared moduli)
-    launch_multi_dot(g.A.get(), g.mg * g.ng, 1, g.A.get(), g.mg * g.ng, partial.get(), dcoef.get(), s);
-    cplx wsum;
-    HIP_CHECK(hipMemcpyAsync(&wsum, dcoef.get(), sizeof(cplx), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    g.weight = wsum.re;
+    // group weights (sums of squared moduli)
+    if (!wjobs.empty()) {
+      const int nb = static_cast<int>(std::min<int64_t>(1024, std::max<int64_t>(1, amax / 4096)));
+      DevBuf<WeightJob> dw(wjobs.size());
+      dw.upload(wjobs.data(), wjobs.size(), s);
+      DevBuf<double> dp(wjobs.size() * static_cast<size_t>(nb));
+      hipLaunchKernelGGL(weight_kernel, dim3(nb, wjobs.size()), dim3(256), 0, s, dw.get(), dp.get());
+      HIP_CHECK(hipGetLastError());
+      std::vector<double> hp(wjobs.size() * static_cast<size_t>(nb));
+      HIP_CHECK(hipMemcpyAsync(hp.data(), dp.get(), hp.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipStreamSynchronize(s));
+      for (size_t q = 0; q < wgroups.size(); ++q)
+        for (int k = 0; k < nb; ++k) wgroups[q]->weight += hp[q * nb + k];
+    }
+  }
+  for (size_t gi = 0; gi < glist.size(); ++gi) {
+    Group& g = *glist[gi];
+    if (g.mg == 0 || g.ng == 0) continue;
     if (g.weight <= eps * eps) continue;                  // empty block: skipped
     // a large block of which at most D values can be kept: leading values
     // only (randomized subspace iteration, accepted on its Ritz residuals)
@@ -393,6 +448,46 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     pending.push_back(Pending{&g, 0, 0, 0, 0.0, false, true});
   }
 
+  // ---- small and middle full decompositions: Jacobi, all in one go ----------
+  DevBuf<cplx> uvbuf;
+  {
+    std::vector<JacobiItem> items;
+    std::vector<size_t> which;
+    int64_t uv = 0;
+    for (size_t q = 0; q < pending.size(); ++q) {
+      Group& g = *pending[q].g;
+      if (!pending[q].full || !jacobi_svd_fits(g.mg, g.ng) || !std::isfinite(g.weight)) continue;
+      which.push_back(q);
+      uv += (g.mg + g.ng) * std::min(g.mg, g.ng);
+    }
+    if (!which.empty()) {
+      const auto t1 = std::chrono::steady_clock::now();
+      if (!values_only) uvbuf.alloc(static_cast<size_t>(uv));
+      cplx* at = uvbuf.get();
+      for (size_t q : which) {
+        Group& g = *pending[q].g;
+        g.k = std::min(g.mg, g.ng);
+        if (!values_only) {
+          g.Up = at;
+          g.Vp = at + g.mg * g.k;
+          at += (g.mg + g.ng) * g.k;
+        }
+        items.push_back(JacobiItem{g.A, g.mg, g.ng, g.weight, g.Up, g.Vp, &g.S});
+      }
+      const std::vector<char> ok = jacobi_svd(ctx, items);
+      std::vector<Pending> rest;
+      for (size_t q = 0, i = 0; q < pending.size(); ++q) {
+        const bool mine = i < which.size() && which[i] == q;
+        if (!(mine && ok[i])) rest.push_back(pending[q]);
+        if (mine) ++i;
+      }
+      if (trace)
+        std::fprintf(stderr, "svd_truncate: %zu of %zu blocks by Jacobi, %.6f s\n", pending.size() - rest.size(),
+                     pending.size(), std::chrono::duration<double>(std::chrono::steady_clock::now() - t1).count());
+      pending.swap(rest);
+    }
+  }
+
   // ---- decompositions --------------------------------------------------------
   // Two lanes: the context's stream and rocBLAS handle, and an auxiliary
   // pair driven from a second host thread, pull the decompositions from one
@@ -407,7 +502,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     std::vector<double> S;
     int rounds = 0;
     const auto t0 = std::chrono::steady_clock::now();
-    pj.ok = truncated_svd(lane, g.A.get(), g.mg, g.ng, pj.kk, pj.ncheck, pj.tol, 24, S, g.U, g.Vh, &rounds,
+    pj.ok = truncated_svd(lane, g.A, g.mg, g.ng, pj.kk, pj.ncheck, pj.tol, 24, S, g.U, g.Vh, &rounds,
                           &g.last_res, pj.naccept, &g.res);
     HIP_CHECK(hipStreamSynchronize(lane.stream));
     if (trace)
@@ -417,6 +512,8 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
                    static_cast<long long>(pj.naccept), pj.ok ? "accepted" : "not accepted", rounds,
                    std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
     if (pj.ok) {
+      g.Up = g.U.get();
+      g.Vp = g.Vh.get();
       g.S = std::move(S);
       g.k = pj.kk;
       g.kk = pj.kk;
@@ -547,8 +644,10 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
       if (g->nver < nver) {
         std::vector<double> S;
         int rounds = 0;
-        if (truncated_svd(ctx, g->A.get(), g->mg, g->ng, g->kk, nver, tol, 24, S, g->U, g->Vh, &rounds,
+        if (truncated_svd(ctx, g->A, g->mg, g->ng, g->kk, nver, tol, 24, S, g->U, g->Vh, &rounds,
                           &g->last_res, nver, &g->res)) {
+          g->Up = g->U.get();
+          g->Vp = g->Vh.get();
           g->S = std::move(S);
           g->nver = nver;
           double kept = 0.0;
@@ -574,7 +673,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
         ctx.svd_kept_hint[std::make_pair(std::array<int64_t, 3>{glist[gi]->mg, glist[gi]->ng, glist[gi]->kk},
                                          glist[gi]->q)] = kept_of[gi];
   }
-  for (Group* g : glist) g->A.reset();
+  abuf.reset();
   values.clear();
   for (size_t i = 0; i < length; ++i) values.push_back(all[i].v);
   if (values_only) return;
@@ -656,7 +755,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
       for (auto li : kept[ub[bi].g]) flat.push_back(li);
       at.push_back({a, c});
       GatherJob j{};
-      j.in = reinterpret_cast<const double2*>(g.U.get());
+      j.in = reinterpret_cast<const double2*>(g.Up);
       j.out = reinterpret_cast<double2*>(U->data.get() + U->blocks[bi].offset);
       j.M = g.rows[t].size;
       j.N = static_cast<int64_t>(kept[ub[bi].g].size());
@@ -676,7 +775,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
       for (int64_t j = 0; j < g.cols[t].size; ++j) flat.push_back(g.cmap[g.coff[t] + j]);
       at.push_back({a, c});
       GatherJob j{};
-      j.in = reinterpret_cast<const double2*>(g.Vh.get());
+      j.in = reinterpret_cast<const double2*>(g.Vp);
       j.out = reinterpret_cast<double2*>(Vd->data.get() + Vd->blocks[bi].offset);
       j.M = static_cast<int64_t>(kept[vb[bi].g].size());
       j.N = g.cols[t].size;

@@ -1,0 +1,69 @@
+"""GPU: the Jacobi decompositions behind the blockwise SVD, at the sizes where
+they change form (one workgroup in LDS up to 69 square, block Jacobi beyond,
+column blocks of 16 with padding, row chunks of 64), against numpy.
+
+A backward-stable SVD of an m x n matrix is off by a small multiple of
+eps sqrt(max(m, n)) |A|; with sizes up to 260 that stays below 1e-13 |A| for
+the values and the reconstruction, and 1e-12 for the vectors' orthonormality.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _svd(ctx, A):
+    import chainamps_amd as cam
+    from chainamps_amd.capi import IndexDesc
+    from chainamps_amd.workloads import tensor_from_dense
+    idx = [IndexDesc(True, False, np.zeros((A.shape[0], 1), int)),
+           IndexDesc(False, False, np.zeros((A.shape[1], 1), int))]
+    U, s, Vd, disc = cam.svd_truncate(tensor_from_dense(ctx, [0], idx, 1, A), 0, 0.0)
+
+    def dense(T):
+        rows, cols, p, i, x = T.to_csc()
+        m = np.zeros((rows, cols), complex)
+        m[i, np.repeat(np.arange(cols), np.diff(p))] = x
+        return m
+    return dense(U), s, dense(Vd)
+
+
+def _check(ctx, A):
+    U, s, Vd = _svd(ctx, A)
+    ref = np.linalg.svd(A, compute_uv=False)
+    nrm = np.linalg.norm(A, 2)
+    k = len(ref)
+    assert len(s) == k
+    assert np.all(np.diff(s) <= 0)
+    assert np.abs(s - ref).max() <= 1e-13 * nrm
+    assert np.linalg.norm((U * s) @ Vd - A, 2) <= 1e-13 * nrm
+    assert np.abs(U.conj().T @ U - np.eye(k)).max() <= 1e-12
+    assert np.abs(Vd @ Vd.conj().T - np.eye(k)).max() <= 1e-12
+
+
+def _rand(rng, *shape):
+    return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 7), (9, 1), (2, 2), (5, 3), (16, 17), (33, 40), (69, 69), (70, 70), (30, 200),
+                                 (200, 30), (64, 65), (129, 96), (97, 130), (80, 300), (192, 192), (260, 257)])
+@pytest.mark.parametrize("graded", [False, True])
+def test_jacobi_sizes(ctx, m, n, graded):
+    print(f"case jacobi m={m} n={n} graded={graded}", flush=True)
+    rng = np.random.default_rng(1000 * m + n)
+    A = _rand(rng, m, n)
+    if graded:      # a decaying spectrum on both sides, as a bond's wavefunction has
+        A = (A * np.exp(-rng.permutation(n) * 12.0 / n)) * np.exp(-rng.permutation(m) * 9.0 / m)[:, None]
+    _check(ctx, A)
+
+
+@pytest.mark.parametrize("n", [24, 69, 100])
+@pytest.mark.parametrize("rank", [1, 5])
+def test_jacobi_rank_deficient(ctx, n, rank):
+    """Null directions come back orthonormal too (the first sites of a
+    product state)."""
+    print(f"case jacobi_rank_deficient n={n} rank={rank}", flush=True)
+    rng = np.random.default_rng(n + rank)
+    _check(ctx, _rand(rng, n, rank) @ _rand(rng, rank, n))
+    # exactly dependent columns: exact zeros appear during the rotations
+    _check(ctx, np.tile(_rand(rng, n, 1), (1, n)) * np.where(np.arange(n) % 2, -1.0, 1.0))
