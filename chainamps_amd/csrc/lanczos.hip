@@ -14,8 +14,8 @@
 // kept fully orthogonal: each new vector is first projected off the last
 // two basis vectors (the large alpha and beta components of the three-term
 // recurrence), then off the whole basis in one classical Gram-Schmidt pass
-// (FP64 sums); the tridiagonal eigenproblem is solved in FP64 on the device
-// with rocSOLVER dsteqr.
+// (FP64 sums); the tridiagonal eigenproblem (at most 63 rows) is solved in
+// FP64 on the host.
 //
 // Mixed precision: each restart starts from the FP64 Ritz vector x, whose
 // FP64 matvec gives the exact Rayleigh quotient and residual r; the Krylov
@@ -24,7 +24,6 @@
 // decreasing; when it stalls, or once it is within 1e3*eps*|theta|, the
 // remaining restarts run in FP64.
 #include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <cmath>
@@ -88,8 +87,6 @@ struct Lanczos {
   float2* w32 = nullptr;
   DevBuf<cplx> coef, partial;
   DevBuf<cplx> C1, C2, Nrm, Dec;   // per-step projection coefficients, norms, decisions
-  DevBuf<double> dD, dE, dC;
-  DevBuf<int> dinfo;
   hipGraphExec_t cycle_exec[2] = {nullptr, nullptr};
   bool use_graphs = true;
   int mv64 = 0, mv32 = 0;
@@ -108,10 +105,6 @@ struct Lanczos {
     C2.alloc(64 * 64);
     Nrm.alloc(64);
     Dec.alloc(64);
-    dD.alloc(64);
-    dE.alloc(64);
-    dC.alloc(64 * 64);
-    dinfo.alloc(1);
     const char* e = std::getenv("CAM_NO_GRAPH");
     use_graphs = !(e && *e && *e != '0');
   }
@@ -261,30 +254,6 @@ struct Lanczos {
     }
     return tot;
   }
-  // lowest eigenpair of the symmetric tridiagonal (alpha, beta) on the device
-  double tridiag_lowest(const std::vector<double>& a, const std::vector<double>& b, std::vector<double>& vec) {
-    const int k = static_cast<int>(a.size());
-    rocblas_handle h = static_cast<rocblas_handle>(H.ctx->blas_handle());
-    std::vector<double> e(std::max(k - 1, 1), 0.0);
-    for (int i = 0; i + 1 < k; ++i) e[i] = b[i];
-    HIP_CHECK(hipMemcpyAsync(dD.get(), a.data(), k * sizeof(double), hipMemcpyHostToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(dE.get(), e.data(), e.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    const rocblas_status st =
-        rocsolver_dsteqr(h, rocblas_evect_tridiagonal, k, dD.get(), dE.get(), dC.get(), k, dinfo.get());
-    CAM_REQUIRE(st == rocblas_status_success, "rocsolver_dsteqr failed");
-    std::vector<double> evals(k), C(static_cast<size_t>(k) * k);
-    int info = 0;
-    HIP_CHECK(hipMemcpyAsync(evals.data(), dD.get(), k * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(C.data(), dC.get(), C.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(&info, dinfo.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    CAM_REQUIRE(info == 0, "tridiagonal eigensolver did not converge");
-    int lo = 0;
-    for (int i = 1; i < k; ++i)
-      if (evals[i] < evals[lo]) lo = i;
-    vec.assign(C.begin() + static_cast<int64_t>(lo) * k, C.begin() + static_cast<int64_t>(lo + 1) * k);
-    return evals[lo];
-  }
 };
 
 }  // namespace
@@ -433,7 +402,7 @@ double lanczos_lowest(Heff& H, cplx* xout, bool have_start, bool converge, doubl
     }
     std::vector<double> svec;
     beta.resize(k, 0.0);
-    const double th = L.tridiag_lowest(alpha, beta, svec);
+    const double th = tridiagonal_lowest(alpha, beta, svec);
     const double ritz_res = invariant ? 0.0 : std::fabs(beta[k - 1] * svec[k - 1]);
     std::vector<std::complex<double>> cs(k);
     for (int j = 0; j < k; ++j) cs[j] = svec[j];
@@ -470,12 +439,6 @@ double lanczos_lowest(Heff& H, cplx* xout, bool have_start, bool converge, doubl
 
 namespace {
 
-__global__ void unit_vector_kernel(double2* x, int64_t n, int64_t j) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x)
-    x[i] = make_double2(i == j ? 1.0 : 0.0, 0.0);
-}
-
 // TranslationBlock<DenseMatrix>::TranslateRows cut (sparse_interface.hpp:414-425):
 // entries with |x| < SPARSETOL are not stored
 __global__ void cut_small_kernel(const double2* __restrict__ x, double2* __restrict__ y, int64_t n, double tol) {
@@ -489,31 +452,33 @@ __global__ void cut_small_kernel(const double2* __restrict__ x, double2* __restr
 }  // namespace
 
 // Dense branch of TwoVertexComponents::HED (DMRG_routines.cpp:850-858): the
-// whole H_eff is formed (column j = H_eff e_j, in the block layout, which is
-// a permutation of the reference's allowed-index order) and diagonalised
-// by hermitian_eig; the lowest eigenvector is returned with entries
-// below SPARSETOL cut and no phase gauge, as the reference's LAPACK path.
+// whole H_eff is formed (in the block layout, a permutation of the reference's
+// allowed-index order) and its lowest eigenpair computed: by Lanczos on the
+// dense matrix, or, should that not reach rounding level, by the full
+// hermitian_eig.  The eigenvector is returned with entries below SPARSETOL
+// cut and no phase gauge, as the reference's LAPACK path.
 double dense_lowest(Heff& H, cplx* xout, double* info) {
   const int64_t n = H.n;
   CAM_REQUIRE(n > 0 && n <= kSparseThreshold, "dense eigensolver: size out of range");
   hipStream_t s = H.ctx->stream;
-  DevBuf<cplx> A(static_cast<size_t>(n) * n), e(n);
-  DevBuf<double> D(n);
+  DevBuf<cplx> A(static_cast<size_t>(n) * n), x(n);
   const int grid = static_cast<int>((n + 255) / 256);
-  for (int64_t j = 0; j < n; ++j) {
-    hipLaunchKernelGGL(unit_vector_kernel, dim3(grid), dim3(256), 0, s, reinterpret_cast<double2*>(e.get()), n, j);
-    HIP_CHECK(hipGetLastError());
-    H.apply(e.get(), A.get() + j * n, 0);
+  dense_heff(H, A.get());
+  double e0 = 0.0;
+  const cplx* v = x.get();
+  if (!hermitian_lowest(*H.ctx, A.get(), n, &e0, x.get())) {
+    DevBuf<double> D(n);
+    hermitian_eig(*H.ctx, A.get(), n, D.get());
+    HIP_CHECK(hipMemcpyAsync(&e0, D.get(), sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+    v = A.get();
   }
-  hermitian_eig(*H.ctx, A.get(), n, D.get());
-  hipLaunchKernelGGL(cut_small_kernel, dim3(grid), dim3(256), 0, s, reinterpret_cast<const double2*>(A.get()),
+  hipLaunchKernelGGL(cut_small_kernel, dim3(grid), dim3(256), 0, s, reinterpret_cast<const double2*>(v),
                      reinterpret_cast<double2*>(xout), n, std::numeric_limits<double>::epsilon());
   HIP_CHECK(hipGetLastError());
   DevBuf<cplx> partial(static_cast<size_t>(multi_dot_blocks(n)) * 64), nrm(1);
   launch_multi_dot(xout, n, 1, xout, n, partial.get(), nrm.get(), s);
-  double e0 = 0.0;
   cplx nx{0.0, 0.0};
-  HIP_CHECK(hipMemcpyAsync(&e0, D.get(), sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipMemcpyAsync(&nx, nrm.get(), sizeof(cplx), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   CAM_REQUIRE(std::fabs(nx.re - 1.0) < 1e-6, "dense eigensolver returned a vector that is not normalised");

@@ -19,6 +19,13 @@ double lanczos_lowest(Heff& H, cplx* x, bool have_start, bool converge, double t
 // dispatcher that picks it, as TwoVertexComponents::HED does.
 constexpr int64_t kSparseThreshold = 1000;
 double dense_lowest(Heff& H, cplx* x, double* info);
+// The dense H_eff (n x n, column-major, block layout), and the lowest
+// eigenpair of a dense Hermitian matrix of that size; false when the pair
+// does not meet its residual test.
+void dense_heff(Heff& H, cplx* A);
+bool hermitian_lowest(Ctx& ctx, const cplx* A, int64_t n, double* e, cplx* x);
+// lowest eigenpair of a symmetric tridiagonal matrix (host)
+double tridiagonal_lowest(const std::vector<double>& a, const std::vector<double>& b, std::vector<double>& vec);
 double eigs_lowest(Heff& H, cplx* x, bool have_start, bool converge, double tol, int ncv, bool mixed,
                    double* info);
 void gauge_fix(cplx* x, int64_t n, hipStream_t s);
