@@ -19,6 +19,7 @@
 #include <array>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -463,130 +464,172 @@ __global__ __launch_bounds__((Waves<R, TM, TN>::kThreads)) void grouped_gemm_ker
   }
 }
 
-// Skinny problems (N <= kSkinnyN, short segments, A M-contiguous): the W
-// stages of small QN sectors, where a 16x16 MFMA fragment would be mostly
-// padding.  One thread per output row accumulates its N outputs in
-// registers.  Per work item the K x N blocks of B of all the problem's
-// segments are staged in LDS once (every thread reads the same element: a
-// broadcast), and the segments' k steps are flattened into one table of
-// (A column address, B row, operand flags), so the loop keeps eight
-// coalesced A loads in flight across segment boundaries with no barrier.
-// A is read once per problem and C written once: bound by HBM like the
-// copy it nearly is.
-template <typename R>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmProb* __restrict__ probs,
-                                                          const GemmSeg* __restrict__ segs,
-                                                          const GemmTile* __restrict__ items, int nitems,
-                                                          GemmBases bases) {
+// Row pass: `rows` rows of nin input columns times an nin x nout matrix, for
+// N <= 16 problems with short segments (the W stages and environments of
+// small QN sectors), where an output tile per problem would be mostly padding
+// and every output channel would read the input rows again.
+// Bound by HBM: per row (nin + nout) elements move for at most 64 x 64
+// complex products, which take as long on the matrix cores; so all problems
+// that read the same columns share a pass (a U(1) MPO with six channels and
+// sectors of 4-5 levels: one pass of 27 x 27 instead of six problems of
+// 27 x 5), and a wave streams 16 rows at a time from memory straight into
+// MFMA operands, eight k steps (8 KB in FP64) in flight, without LDS or
+// barriers.  The matrix is staged in LDS once per item, gathered by all
+// threads at once through the pass's tables; rows run on over the batch
+// members (they share B), so small row counts still fill the wave.
+// U(1) chain, d=32, chi=1024: W stages 9.6 / 9.2 ms with one thread per row
+// and problem -> 3.63 / 3.55 ms (12.9 GB to move each: 3.6 TB/s; a large copy
+// reaches 4.8); chain d=64, chi=32: stage R (16 x 16 blocks, 1024 batch
+// members) 0.74 -> 0.035 ms; spin chain chi=16: matvec 31 -> 21 us.
+constexpr int kRowThreads = 256;
+constexpr int kRowWaves = kRowThreads / 64;
+
+template <typename R, int NT>
+__device__ __forceinline__ void row_pass(const RowItem& it, const typename CT<R>::T* sB,
+                                         const typename CT<R>::T* const* sInP, const int64_t* sInS,
+                                         typename CT<R>::T* const* sOutP, const int64_t* sOutS) {
   using C = typename CT<R>::T;
-  __shared__ R sBr[kSkinnyB], sBi[kSkinnyB];
-  __shared__ const C* sStepA[kSkinnySteps];    // A column of the step, batch and k applied
-  __shared__ int sStepB[kSkinnySteps];         // first element of its B row in sBr / sBi
-  __shared__ int sStepF[kSkinnySteps];         // segment flags
-  __shared__ int sSegK[kSkinnySegs], sSegOff[kSkinnySegs], sSegStep[kSkinnySegs];
-  const int tid = threadIdx.x;
-  // XCD-aware order, as for the tiles: consecutive items (the problems of
-  // one row group over the same rows, which read the same A rows) go to
-  // workgroups of one XCD, whose L2 then serves the repeated reads
-  const int Gd = gridDim.x;
-  const int v0 = (Gd % kXcds == 0) ? (blockIdx.x % kXcds) * (Gd / kXcds) + blockIdx.x / kXcds : blockIdx.x;
-  for (int it = v0; it < nitems; it += Gd) {
-    const GemmTile w = cload(items + it);
-    const GemmProb P = cload(probs + w.prob);
-    const int M = P.M, N = P.N, ns = P.nseg;
-    __syncthreads();   // the previous item's tables are no longer read
-    if (tid < ns) sSegK[tid] = cload(segs + P.seg0 + tid).K;
-    __syncthreads();
-    if (tid == 0) {
-      int off = 0, st = 0;
-      for (int j = 0; j < ns; ++j) {
-        sSegOff[j] = off;
-        sSegStep[j] = st;
-        off += sSegK[j] * N;
-        st += sSegK[j];
+  using V = typename NV<C>::T;
+  using acc_t = typename Mf<R>::acc;
+  constexpr int NP = 16 * NT, U = 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int fr = lane & 15, fk = lane >> 4;
+  const int nks = (it.nin + 3) / 4;
+  for (int c0 = wave * 16; c0 < it.rows; c0 += kRowWaves * 16) {
+    // rows past the item repeat its last one and are not stored
+    const bool live = c0 + fr < it.rows;
+    const uint32_t t = static_cast<uint32_t>(it.m0) + static_cast<uint32_t>(min(c0 + fr, it.rows - 1));
+    const uint32_t q = t / static_cast<uint32_t>(it.M);
+    const int64_t b = it.batch0 + static_cast<int64_t>(q);
+    const int64_t m = t - q * static_cast<uint32_t>(it.M);
+    acc_t cr[NT], ci[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) cr[j][v] = ci[j][v] = R(0);
+    for (int k0 = 0; k0 < nks; k0 += U) {
+      V a[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = min((k0 + u) * 4 + fk, it.nin - 1);
+        a[u] = *(const __attribute__((address_space(1))) V*)(sInP[k] + (b * sInS[k] + m));
       }
-    }
-    __syncthreads();
-    int nsteps = 0;
-    for (int j = 0; j < ns; ++j) nsteps += sSegK[j];
-    // B blocks and the step table of every segment
-    for (int j = 0; j < ns; ++j) {
-      const GemmSeg G = cload(segs + P.seg0 + j);
-      const int asp = (G.flags >> 8) & 15, bsp = (G.flags >> 12) & 15;
-      const C* Ab = (asp ? reinterpret_cast<const C*>(bases.p[asp]) + reinterpret_cast<intptr_t>(G.A)
-                         : reinterpret_cast<const C*>(G.A)) +
-                    static_cast<int64_t>(w.batch) * G.bsA;
-      const C* Bb = (bsp ? reinterpret_cast<const C*>(bases.p[bsp]) + reinterpret_cast<intptr_t>(G.B)
-                         : reinterpret_cast<const C*>(G.B)) +
-                    static_cast<int64_t>(w.batch) * G.bsB;
-      const bool cB = G.flags & kSegConjB, bnc = G.flags & kSegBNContig;
-      const int K = G.K, off = sSegOff[j], st = sSegStep[j];
-      for (int e = tid; e < K * N; e += 256) {
-        const int k = e / N, n = e % N;
-        const C b = gload(Bb + (bnc ? static_cast<int64_t>(k) * G.ldB + n : k + static_cast<int64_t>(n) * G.ldB));
-        sBr[off + e] = b.x;
-        sBi[off + e] = cB ? -b.y : b.y;
-      }
-      if (tid < K) {
-        sStepA[st + tid] = Ab + static_cast<int64_t>(tid) * G.csA;
-        sStepB[st + tid] = off + tid * N;
-        sStepF[st + tid] = G.flags;
-      }
-    }
-    __syncthreads();
-    const int m = w.m0 + tid;
-    if (m >= M) continue;
-    R accr[kSkinnyN], acci[kSkinnyN];
 #pragma unroll
-    for (int n = 0; n < kSkinnyN; ++n) accr[n] = acci[n] = R(0);
-    for (int j0 = 0; j0 < nsteps; j0 += 8) {
-      C a[8];
+      for (int u = 0; u < U; ++u) {
+        if (k0 + u >= nks) break;
+        const int k = (k0 + u) * 4 + fk;
+        const bool in = k < it.nin;
+        const R ar = in ? a[u].x : R(0);
+        const R ai = in ? (it.conjA ? -a[u].y : a[u].y) : R(0);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) a[u] = gload(sStepA[j0 + u < nsteps ? j0 + u : j0] + m);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (j0 + u >= nsteps) break;
-        const int j = j0 + u, fl = sStepF[j], bo = sStepB[j];
-        const R xr = a[u].x, xi = (fl & kSegConjA) ? -a[u].y : a[u].y;
-#pragma unroll
-        for (int n = 0; n < kSkinnyN; ++n) {
-          if (n >= N) break;
-          const R br = sBr[bo + n], bi = sBi[bo + n];
-          accr[n] += xr * br - xi * bi;
-          acci[n] += xr * bi + xi * br;
+        for (int j = 0; j < NT; ++j) {
+          const C bv = sB[k * NP + j * 16 + fr];
+          cr[j] = Mf<R>::mma(bv.x, ar, cr[j]);
+          ci[j] = Mf<R>::mma(bv.x, ai, ci[j]);
+          cr[j] = Mf<R>::mma(-bv.y, ai, cr[j]);
+          ci[j] = Mf<R>::mma(bv.y, ar, ci[j]);
         }
       }
     }
-    C* Cp = (P.cspace ? reinterpret_cast<C*>(const_cast<void*>(bases.p[P.cspace])) + reinterpret_cast<intptr_t>(P.C)
-                      : reinterpret_cast<C*>(P.C)) +
-            static_cast<int64_t>(w.batch) * P.bsC + m;
+    if (live) {
 #pragma unroll
-    for (int n = 0; n < kSkinnyN; ++n) {
-      if (n >= N) break;
-      C* dst = Cp + static_cast<int64_t>(n) * P.csC;
-      C val;
-      val.x = accr[n];
-      val.y = acci[n];
-      if (P.beta) {
-        const C old = gload(dst);
-        val.x += old.x;
-        val.y += old.y;
-      }
-      gstore(dst, val);
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int n = j * 16 + Mf<R>::row(fk, v);
+          if (n >= it.nout) continue;
+          C* dst = sOutP[n] + (b * sOutS[n] + m);
+          C val;
+          val.x = cr[j][v];
+          val.y = ci[j][v];
+          if (it.beta) {
+            const C old = gload(dst);
+            val.x += old.x;
+            val.y += old.y;
+          }
+          gstore(dst, val);
+        }
     }
   }
 }
 
 template <typename R>
-void launch_skinny(const GemmPlan& plan, const LaunchCfg& c, hipStream_t s, int grid_limit, const GemmBases& bases) {
-  const int n = static_cast<int>(plan.skinny.size());
+__global__ __launch_bounds__(kRowThreads) void row_gemm_kernel(const RowItem* __restrict__ items, int nitems,
+                                                               const RowIn* __restrict__ ins,
+                                                               const RowOut* __restrict__ outs,
+                                                               const RowBlk* __restrict__ blks, GemmBases bases) {
+  using C = typename CT<R>::T;
+  extern __shared__ __align__(16) char smem[];
+  C* sB = reinterpret_cast<C*>(smem);          // [padded nin][16 NT]
+  __shared__ const C* sInP[kRowIn];
+  __shared__ int64_t sInS[kRowIn];
+  __shared__ int sInB[kRowIn];                 // first block of the column's segment
+  __shared__ int sInK[kRowIn];
+  __shared__ C* sOutP[kRowOut];
+  __shared__ int64_t sOutS[kRowOut];
+  __shared__ int sOutB[kRowOut], sOutN[kRowOut];
+  const int tid = threadIdx.x;
+  // XCD-aware order, as for the tiles: consecutive items (passes over the
+  // same rows) go to workgroups of one XCD, whose L2 serves repeated reads
+  const int Gd = gridDim.x;
+  const int v0 = (Gd % kXcds == 0) ? (blockIdx.x % kXcds) * (Gd / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+  for (int i = v0; i < nitems; i += Gd) {
+    const RowItem it = cload(items + i);
+    const C* ab = it.aspace ? reinterpret_cast<const C*>(bases.p[it.aspace]) : nullptr;
+    const C* bb = it.bspace ? reinterpret_cast<const C*>(bases.p[it.bspace]) : nullptr;
+    C* cb = it.cspace ? reinterpret_cast<C*>(const_cast<void*>(bases.p[it.cspace])) : nullptr;
+    if (i != v0) __syncthreads();              // the previous item's tables are no longer read
+    if (tid < it.nin) {
+      const RowIn e = ins[it.in0 + tid];
+      sInP[tid] = (it.aspace ? ab + e.off : reinterpret_cast<const C*>(e.off)) + e.kcs;
+      sInS[tid] = e.bs;
+      sInB[tid] = it.blk0 + e.seg * it.nprob;
+      sInK[tid] = e.k;
+    } else if (tid >= kRowThreads - kRowOut && tid - (kRowThreads - kRowOut) < it.nout) {
+      const int n = tid - (kRowThreads - kRowOut);
+      const RowOut e = outs[it.out0 + n];
+      sOutP[n] = (it.cspace ? cb + e.off : reinterpret_cast<C*>(e.off)) + e.ncs;
+      sOutS[n] = e.bs;
+      sOutB[n] = e.prob;
+      sOutN[n] = e.n;
+    }
+    __syncthreads();
+    const int nt = (it.nout + 15) / 16, np = 16 * nt;
+    const int tot = (it.nin + 3) / 4 * 4 * np;
+    for (int e = tid; e < tot; e += kRowThreads) {
+      const int k = e / np, n = e % np;
+      C v;
+      v.x = v.y = R(0);
+      if (k < it.nin && n < it.nout) {
+        const RowBlk B = blks[sInB[k] + sOutB[n]];
+        const C* Bp = it.bspace ? bb + B.off : reinterpret_cast<const C*>(B.off);
+        const int64_t kk = sInK[k], nn = sOutN[n];
+        v = gload(Bp + ((B.flags & kSegBNContig) ? kk * B.ld + nn : kk + nn * B.ld));
+        if (B.flags & kSegConjB) v.y = -v.y;
+      }
+      sB[e] = v;
+    }
+    __syncthreads();
+    if (nt == 1) row_pass<R, 1>(it, sB, sInP, sInS, sOutP, sOutS);
+    else if (nt == 2) row_pass<R, 2>(it, sB, sInP, sInS, sOutP, sOutS);
+    else if (nt == 3) row_pass<R, 3>(it, sB, sInP, sInS, sOutP, sOutS);
+    else row_pass<R, 4>(it, sB, sInP, sInS, sOutP, sOutS);
+  }
+}
+
+template <typename R>
+void launch_rows(const GemmPlan& plan, hipStream_t s, int grid_limit, const GemmBases& bases) {
+  const int n = static_cast<int>(plan.rows.size());
   if (!n) return;
   static int cus = device_cu_count();
   int grid = std::min(n, cus * 8);
   if (grid_limit > 0) grid = std::min(grid, grid_limit);
-  (void)c;
-  hipLaunchKernelGGL((skinny_gemm_kernel<R>), dim3(grid), dim3(256), 0, s, plan.d_probs.get(), plan.d_segs.get(),
-                     plan.d_skinny.get(), n, bases);
+  const size_t lds = static_cast<size_t>(plan.row_lds) * sizeof(typename CT<R>::T);
+  const RowIn* in = reinterpret_cast<const RowIn*>(plan.d_rows.get());
+  const RowOut* out = reinterpret_cast<const RowOut*>(in + plan.row_in.size());
+  const RowBlk* blk = reinterpret_cast<const RowBlk*>(out + plan.row_out.size());
+  const RowItem* items = reinterpret_cast<const RowItem*>(blk + plan.row_blk.size());
+  hipLaunchKernelGGL((row_gemm_kernel<R>), dim3(grid), dim3(kRowThreads), lds, s, items, n, in, out, blk, bases);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -691,34 +734,138 @@ void GemmPlan::build_tiles() {
   if (cfg[1].tile_mode != cfg[0].tile_mode) build_tiles_mode(cfg[1].tile_mode);
 }
 
-static bool skinny_eligible(const GemmPlan& plan, const GemmProb& p) {
+// Row pass or tiles: N <= 16 and K <= 32 per segment (see GemmPlan::rows).
+// Below the line the tiles lose: U(1) chi=1024 W stages 15.4 ms against 3.6,
+// spin chain chi=200 W stages 50 us against 9, chain d=64 chi=32 stage R 0.128
+// ms against 0.035.  Above it the passes do: they take four products where
+// the tiles take three and re-read B per 16 rows; with N up to 32 the W stages
+// of the d=64 chain run at 24 TFLOP/s against 44-55 (chi=64, 97, 500), FP32 54
+// against 90 (chi=256).
+static bool row_eligible(const GemmPlan& plan, const GemmProb& p) {
   static const bool off = [] {
     const char* e = std::getenv("CAM_SKINNY");
     return e && *e == '0';
   }();
-  if (off || p.N > kSkinnyN || p.nseg == 0 || p.nseg > kSkinnySegs) return false;
-  int64_t steps = 0;
+  if (off || p.N > kRowN || p.nseg == 0 || p.M <= 0 || p.N <= 0) return false;
+  int64_t k = 0;
+  const GemmSeg& g0 = plan.segs[p.seg0];
   for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) {
     const GemmSeg& g = plan.segs[s];
-    if (g.K > kSkinnyK || (g.flags & kSegAKContig)) return false;
-    steps += g.K;
+    if (g.K > kRowK || (g.flags & kSegAKContig) || ((g.flags ^ g0.flags) >> 8)) return false;
+    if (g.bsB && p.batch > 1) return false;   // one matrix for all rows
+    k += g.K;
   }
-  // the step table and every B block fit the kernel's LDS tables
-  return steps <= kSkinnySteps && steps * p.N <= kSkinnyB;
+  return k <= kRowIn;
+}
+
+// Passes: problems with the same rows and the same input columns, up to
+// kRowOut output columns and kRowB matrix elements each.  (Problems with
+// different inputs are not merged: a channel that an output does not read
+// must not reach it, not even as zero times infinity.)
+void GemmPlan::build_rows(const std::vector<int>& eligible) {
+  row_in.clear();
+  row_out.clear();
+  row_blk.clear();
+  rows.clear();
+  row_lds = 0;
+  rows_uploaded = false;
+  if (eligible.empty()) return;
+  struct Pass { std::vector<int> probs; int nout = 0; };
+  std::vector<Pass> passes;
+  std::map<std::vector<int64_t>, int> open;   // input signature -> pass still being filled
+  for (int pi : eligible) {
+    const GemmProb& p = probs[pi];
+    std::vector<int64_t> key{p.M, p.batch, p.beta, p.cspace};
+    int nin = 0;
+    for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) {
+      const GemmSeg& g = segs[s];
+      key.insert(key.end(), {reinterpret_cast<int64_t>(g.A), g.csA, g.bsA, g.K,
+                             g.flags & ~(kSegConjB | kSegBNContig)});
+      nin += g.K;
+    }
+    const int kp = (nin + 3) / 4 * 4;
+    auto it = open.find(key);
+    if (it != open.end()) {
+      const int no = passes[it->second].nout + p.N;
+      if (no > kRowOut || kp * ((no + 15) / 16 * 16) > kRowB) it = open.end();
+    }
+    if (it == open.end()) {
+      open[key] = static_cast<int>(passes.size());
+      passes.emplace_back();
+      it = open.find(key);
+    }
+    passes[it->second].probs.push_back(pi);
+    passes[it->second].nout += p.N;
+  }
+  // rows per item: long enough to pay for staging the matrix, short enough
+  // for several items per compute unit
+  int64_t total = 0;
+  for (const Pass& q : passes) total += int64_t(probs[q.probs[0]].M) * probs[q.probs[0]].batch;
+  int per = 1024;
+  while (per > 16 * kRowWaves && total / per < 2048) per /= 2;
+  struct Key { int64_t g, r0; int pass; };
+  std::vector<std::pair<Key, RowItem>> items;
+  for (size_t qi = 0; qi < passes.size(); ++qi) {
+    const Pass& q = passes[qi];
+    const GemmProb& p0 = probs[q.probs[0]];
+    const GemmSeg& g0 = segs[p0.seg0];
+    RowItem it{};
+    it.in0 = static_cast<int>(row_in.size());
+    it.out0 = static_cast<int>(row_out.size());
+    it.blk0 = static_cast<int>(row_blk.size());
+    for (int j = 0; j < p0.nseg; ++j) {
+      const GemmSeg& g = segs[p0.seg0 + j];
+      for (int k = 0; k < g.K; ++k)
+        row_in.push_back(RowIn{reinterpret_cast<int64_t>(g.A), k * g.csA, g.bsA, j, k});
+      for (int pi : q.probs) {
+        const GemmSeg& gp = segs[probs[pi].seg0 + j];
+        row_blk.push_back(RowBlk{reinterpret_cast<int64_t>(gp.B), static_cast<int32_t>(gp.ldB), gp.flags});
+      }
+    }
+    for (size_t j = 0; j < q.probs.size(); ++j) {
+      const GemmProb& p = probs[q.probs[j]];
+      for (int n = 0; n < p.N; ++n)
+        row_out.push_back(RowOut{reinterpret_cast<int64_t>(p.C), n * p.csC, p.bsC, static_cast<int32_t>(j), n});
+    }
+    it.nin = static_cast<int>(row_in.size()) - it.in0;
+    it.nout = q.nout;
+    it.nprob = static_cast<int>(q.probs.size());
+    it.M = p0.M;
+    it.aspace = (g0.flags >> 8) & 15;
+    it.bspace = (g0.flags >> 12) & 15;
+    it.cspace = p0.cspace;
+    it.conjA = (g0.flags & kSegConjA) ? 1 : 0;
+    it.beta = p0.beta;
+    row_lds = std::max(row_lds, (it.nin + 3) / 4 * 4 * ((it.nout + 15) / 16 * 16));
+    const int64_t all = int64_t(p0.M) * p0.batch;
+    const int64_t g = group[q.probs[0]] >= 0 ? group[q.probs[0]] : -1 - q.probs[0];
+    for (int64_t r0 = 0; r0 < all; r0 += per) {
+      it.batch0 = static_cast<int32_t>(r0 / p0.M);
+      it.m0 = static_cast<int32_t>(r0 % p0.M);
+      it.rows = static_cast<int32_t>(std::min<int64_t>(per, all - r0));
+      items.push_back({Key{g, r0, static_cast<int>(qi)}, it});
+    }
+  }
+  // passes of one row group next to each other at equal rows: they read the
+  // same operand (from one XCD's L2 the second time)
+  std::stable_sort(items.begin(), items.end(), [](const auto& x, const auto& y) {
+    if (x.first.g != y.first.g) return x.first.g < y.first.g;
+    if (x.first.r0 != y.first.r0) return x.first.r0 < y.first.r0;
+    return x.first.pass < y.first.pass;
+  });
+  rows.reserve(items.size());
+  for (auto& e : items) rows.push_back(e.second);
 }
 
 void GemmPlan::build_tiles_mode(int mode) {
   auto& T = tiles[mode];
   for (int t = 0; t < kNumTileShapes; ++t) T[t].clear();
   std::vector<double> cost[kNumTileShapes];
-  skinny.clear();
-  skinny_uploaded = false;
+  std::vector<int> row_probs;
   for (size_t pi = 0; pi < probs.size(); ++pi) {
     const GemmProb& p = probs[pi];
-    if (skinny_eligible(*this, p)) {
-      for (int b = 0; b < p.batch; ++b)
-        for (int m0 = 0; m0 < p.M; m0 += kSkinnyRows)
-          skinny.push_back(GemmTile{static_cast<int32_t>(pi), b, m0, 0});
+    if (row_eligible(*this, p)) {
+      row_probs.push_back(static_cast<int>(pi));
       continue;
     }
     int shape = 0;
@@ -791,16 +938,7 @@ void GemmPlan::build_tiles_mode(int mode) {
     for (auto o : ord) sorted.push_back(T[t][o]);
     T[t].swap(sorted);
   }
-  // skinny items: the problems of one row group (same A rows) next to each
-  // other at equal (batch, m0), so that they run together on one XCD
-  std::stable_sort(skinny.begin(), skinny.end(), [&](const GemmTile& x, const GemmTile& y) {
-    const int64_t gx = group[x.prob] >= 0 ? group[x.prob] : -1 - x.prob;
-    const int64_t gy = group[y.prob] >= 0 ? group[y.prob] : -1 - y.prob;
-    if (gx != gy) return gx < gy;
-    if (x.batch != y.batch) return x.batch < y.batch;
-    if (x.m0 != y.m0) return x.m0 < y.m0;
-    return x.prob < y.prob;
-  });
+  build_rows(row_probs);
   built[mode] = true;
   tiles_uploaded[mode] = false;
 }
@@ -813,10 +951,25 @@ void GemmPlan::upload(hipStream_t s) {
     d_segs.upload(segs.data(), segs.size(), s);
     uploaded = true;
   }
-  if (!skinny_uploaded) {
-    d_skinny.ensure(std::max<size_t>(skinny.size(), 1));
-    d_skinny.upload(skinny.data(), skinny.size(), s);
-    skinny_uploaded = true;
+  if (!rows_uploaded) {
+    if (!rows.empty()) {
+      static_assert(sizeof(RowIn) % 8 == 0 && sizeof(RowOut) % 8 == 0 && sizeof(RowBlk) % 8 == 0,
+                    "the row tables lie one after another");
+      auto words = [](size_t bytes) { return (bytes + 7) / 8; };
+      std::vector<int64_t> h(words(row_in.size() * sizeof(RowIn) + row_out.size() * sizeof(RowOut) +
+                                   row_blk.size() * sizeof(RowBlk) + rows.size() * sizeof(RowItem)));
+      char* q = reinterpret_cast<char*>(h.data());
+      auto put = [&q](const auto& v) {
+        std::memcpy(q, v.data(), v.size() * sizeof(v[0]));
+        q += v.size() * sizeof(v[0]);
+      };
+      put(row_in);
+      put(row_out);
+      put(row_blk);
+      put(rows);
+      d_rows.upload(h, s);
+    }
+    rows_uploaded = true;
   }
   for (int m = 0; m < kTileModes; ++m) {
     if (!built[m] || tiles_uploaded[m]) continue;
@@ -832,8 +985,11 @@ void GemmPlan::clear() {
   probs.clear();
   segs.clear();
   group.clear();
-  skinny.clear();
-  skinny_uploaded = false;
+  row_in.clear();
+  row_out.clear();
+  row_blk.clear();
+  rows.clear();
+  rows_uploaded = false;
   for (int m = 0; m < kTileModes; ++m) {
     for (auto& t : tiles[m]) t.clear();
     built[m] = false;
@@ -958,7 +1114,7 @@ void launch_grouped_gemm(GemmPlan& plan, int precision, hipStream_t s, const Gem
     launch_shape<double, 128, 64>(plan, c, 3, s, grid_limit, b);
     launch_shape<double, 64, 128>(plan, c, 4, s, grid_limit, b);
     launch_shape<double, 128, 32>(plan, c, 5, s, grid_limit, b);
-    launch_skinny<double>(plan, c, s, grid_limit, b);
+    launch_rows<double>(plan, s, grid_limit, b);
   } else {
     launch_shape<float, 64, 64>(plan, c, 0, s, grid_limit, b);
     launch_shape<float, 32, 64>(plan, c, 1, s, grid_limit, b);
@@ -966,7 +1122,7 @@ void launch_grouped_gemm(GemmPlan& plan, int precision, hipStream_t s, const Gem
     launch_shape<float, 128, 64>(plan, c, 3, s, grid_limit, b);
     launch_shape<float, 64, 128>(plan, c, 4, s, grid_limit, b);
     launch_shape<float, 128, 32>(plan, c, 5, s, grid_limit, b);
-    launch_skinny<float>(plan, c, s, grid_limit, b);
+    launch_rows<float>(plan, s, grid_limit, b);
   }
 }
 

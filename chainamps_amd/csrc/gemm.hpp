@@ -67,13 +67,35 @@ struct GemmTile {
   int32_t prob, batch, m0, n0;
 };
 
-// Bounds of the skinny path (see GemmPlan::skinny).
-constexpr int kSkinnyN = 16;       // columns
-constexpr int kSkinnyK = 32;       // K of one segment
-constexpr int kSkinnySegs = 64;    // segments of one problem
-constexpr int kSkinnySteps = 256;  // sum of the segments' K
-constexpr int kSkinnyB = 1024;     // sum of the segments' K x N
-constexpr int kSkinnyRows = 256;
+// Row passes (see GemmPlan::rows).  A pass multiplies rows of `nin` input
+// columns (the A columns of its problems' segments) with an nin x nout matrix
+// (their B blocks) into `nout` output columns (the columns of its problems).
+constexpr int kRowN = 16;       // columns of one problem
+constexpr int kRowK = 32;       // K of one segment
+constexpr int kRowIn = 192;     // input columns of a pass
+constexpr int kRowOut = 64;     // output columns of a pass
+constexpr int kRowB = 3072;     // elements of the padded matrix (LDS)
+
+struct RowIn {                  // one input column
+  int64_t off;                  // segment's A (address or offset, as GemmSeg::A)
+  int64_t kcs, bs;              // column offset in it and batch stride (elements)
+  int32_t seg, k;               // segment of the pass, column of the segment
+};
+struct RowOut {                 // one output column
+  int64_t off, ncs, bs;
+  int32_t prob, n;              // problem of the pass, column of the problem
+};
+struct RowBlk {                 // B block of (segment, problem)
+  int64_t off;
+  int32_t ld, flags;
+};
+struct RowItem {                // rows [.., + rows) of a pass, from row m0 of batch b0
+  int32_t in0, out0, blk0;      // first entries in the tables
+  int32_t nin, nout, nprob;
+  int32_t M, batch0, m0, rows;
+  int32_t aspace, bspace, cspace;
+  int32_t conjA, beta;
+};
 
 // Tile shapes compiled into the kernels (TM x TN per workgroup).
 struct TileShape { int tm, tn; };
@@ -111,14 +133,18 @@ struct GemmPlan {
   bool tiles_uploaded[kTileModes] = {false, false, false};
   LaunchCfg cfg[2];                       // per precision (0 FP64, 1 FP32)
   bool tuned[2] = {false, false};
-  // Problems with at most kSkinnyN columns whose segments all have
-  // K <= kSkinnyK and an M-contiguous A, within the skinny kernel's table
-  // bounds (tiny QN sectors: MFMA tiles would be mostly padding) run in
-  // the skinny kernel instead, one work item per (problem, batch, 256
-  // rows); the list is built with the tiles.
-  std::vector<GemmTile> skinny;
-  DevBuf<GemmTile> d_skinny;
-  bool skinny_uploaded = false;
+  // Problems with at most kRowN columns whose segments all have K <= kRowK
+  // and an M-contiguous A (W stages and environments of small QN sectors: a
+  // tile would be mostly padding) run as row passes: problems that read the
+  // same input columns share a pass, and the rows of all batch members follow
+  // one another.  Tables and items are built with the tiles.
+  std::vector<RowIn> row_in;
+  std::vector<RowOut> row_out;
+  std::vector<RowBlk> row_blk;
+  std::vector<RowItem> rows;
+  int row_lds = 0;                        // largest padded matrix (elements)
+  DevBuf<int64_t> d_rows;                 // all four, in the order in, out, blocks, items
+  bool rows_uploaded = false;
   // Per problem, a row group (-1: none).  Problems of one group read the
   // same A rows (one output per MPO channel from the same operand rows), so
   // their tiles of equal (batch, m0) are ordered next to each other and run
@@ -135,6 +161,8 @@ struct GemmPlan {
   // tiles of the selected policies, LPT-sorted
   void build_tiles();
   void build_tiles_mode(int mode);
+  // tables and items of the row passes over the given problems
+  void build_rows(const std::vector<int>& eligible);
   // Histogram signature: problems bucketed by (log2 M, log2 N, log2 K,
   // batched), weighted by flops (5% steps), plus the precision.
   uint64_t signature(int precision) const;
