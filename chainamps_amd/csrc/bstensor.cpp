@@ -215,6 +215,8 @@ std::vector<cplx> download(const BSTensor& t, hipStream_t s) {
 
 int64_t tensor_to_csc(const BSTensor& t, int64_t cap, int64_t* p, int64_t* ii, double* x,
                       hipStream_t s) {
+  int64_t found = 0;
+  if (tensor_to_csc_device(t, cap, p, ii, x, s, found)) return found;
   std::vector<cplx> h = download(t, s);
   const int n = t.nidx();
   const int64_t rows = t.rows(), cols = t.cols();

@@ -91,6 +91,9 @@ TensorPtr tensor_from_csc(const Rules& rules, std::vector<QIndex> idx, int numro
 // and cap suffices.
 int64_t tensor_to_csc(const BSTensor& t, int64_t cap, int64_t* p, int64_t* i, double* x,
                       hipStream_t s);
+// The same on the device where that pays (csc.hip); false: not done.
+bool tensor_to_csc_device(const BSTensor& t, int64_t cap, int64_t* p, int64_t* i, double* x, hipStream_t s,
+                          int64_t& nnz);
 std::vector<cplx> download(const BSTensor& t, hipStream_t s);
 
 }  // namespace cam
