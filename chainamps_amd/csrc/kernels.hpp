@@ -56,6 +56,13 @@ int multi_dot_blocks(int64_t n);
 // c = V^H w; w -= V c; and w (FP64) += V c.
 void launch_multi_dot32(const float2* V, int64_t ldv, int k, const float2* w, int64_t n, cplx* partial, cplx* c,
                         hipStream_t s);
+// c2 = V^H u and w = u - V c2, |w|^2 to nrm, with u = w - [v_{k-2} v_{k-1}] c1
+// (2 <= k <= 64; c1: the two local coefficients, on the device); partial as
+// for multi dot.
+void launch_gram_schmidt(const cplx* V, int64_t ldv, int k, cplx* w, const cplx* c1, cplx* c2, cplx* nrm, int64_t n,
+                         cplx* partial, hipStream_t s);
+void launch_gram_schmidt32(const float2* V, int64_t ldv, int k, float2* w, const cplx* c1, cplx* c2, cplx* nrm,
+                           int64_t n, cplx* partial, hipStream_t s);
 void launch_multi_axpy32(const float2* V, int64_t ldv, int k, const cplx* c, float2* w, int64_t n, hipStream_t s);
 // c[i] *= w[i], i < k (k <= 64), on the device
 void launch_coef_scale(cplx* c, const cplx* w, int k, hipStream_t s);

@@ -130,9 +130,8 @@ struct Lanczos {
   // catches), so the single full pass suffers no cancellation and restores
   // orthogonality to working precision -- where a full pass applied to
   // H v_j directly cancels |alpha| / beta of the vector and needs a second
-  // pass.  Per step this streams 2j + 15 + ceil((j+1)/8) vectors (the dot
-  // sweeps re-read w once per eight basis vectors) instead of the
-  // 4j + 12 + 2 ceil((j+1)/8) of two full passes.
+  // pass.  Per step this streams 2j + 11 vectors (3 for the local dots, 2j + 6
+  // for both passes, 2 for the normalisation).
   void enqueue_cycle(int prec) {
     const double eps16 = 16 * std::numeric_limits<double>::epsilon();
     if (prec == 1) {
@@ -143,10 +142,7 @@ struct Lanczos {
         cplx* c1 = C1.get() + j * 64;
         cplx* c2 = C2.get() + j * 64;
         launch_multi_dot32(col32(j - 1), n, 2, w32, n, partial.get(), c1 + (j - 1), s);
-        launch_multi_axpy32(col32(j - 1), n, 2, c1 + (j - 1), w32, n, s);
-        launch_multi_dot32(V32, n, j + 1, w32, n, partial.get(), c2, s);
-        launch_multi_axpy32(V32, n, j + 1, c2, w32, n, s);
-        launch_multi_dot32(w32, n, 1, w32, n, partial.get(), Nrm.get() + j, s);
+        launch_gram_schmidt32(V32, n, j + 1, w32, c1 + (j - 1), c2, Nrm.get() + j, n, partial.get(), s);
         const int grid = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(2048, (n + 255) / 256)));
         hipLaunchKernelGGL(lanczos_next_kernel<float2>, dim3(grid), dim3(256), 0, s, w32,
                            j + 1 < m ? col32(j + 1) : nullptr, n, reinterpret_cast<const double2*>(Nrm.get() + j),
@@ -160,13 +156,10 @@ struct Lanczos {
       H.apply(col(j), w.get(), prec);
       cplx* c1 = C1.get() + j * 64;
       cplx* c2 = C2.get() + j * 64;
-      // local pass c = [v_{j-1} v_j]^H w, w -= [v_{j-1} v_j] c; full pass
-      // c = V^H w, w -= V c; then |w|^2
+      // local coefficients [v_{j-1} v_j]^H w; then the local update and the
+      // full pass c = V^H w, w -= V c, with |w|^2
       launch_multi_dot(col(j - 1), n, 2, w.get(), n, partial.get(), c1 + (j - 1), s);
-      launch_multi_axpy(col(j - 1), n, 2, c1 + (j - 1), w.get(), n, s);
-      launch_multi_dot(V.get(), n, j + 1, w.get(), n, partial.get(), c2, s);
-      launch_multi_axpy(V.get(), n, j + 1, c2, w.get(), n, s);
-      launch_multi_dot(w.get(), n, 1, w.get(), n, partial.get(), Nrm.get() + j, s);
+      launch_gram_schmidt(V.get(), n, j + 1, w.get(), c1 + (j - 1), c2, Nrm.get() + j, n, partial.get(), s);
       const int grid = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(2048, (n + 255) / 256)));
       hipLaunchKernelGGL(lanczos_next_kernel<double2>, dim3(grid), dim3(256), 0, s,
                          reinterpret_cast<const double2*>(w.get()),
