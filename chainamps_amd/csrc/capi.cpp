@@ -398,6 +398,7 @@ int cam_heff_set_launch(cam_heff* h, int precision, int algo, int tile_mode, int
   c.tile_mode = tile_mode;
   c.wg_per_cu = wg_per_cu;
   c.kc = kchunk;
+  c.direct = false;
   h->h.set_launch(precision, c);
   CAM_API_END
 }

@@ -633,6 +633,155 @@ void launch_rows(const GemmPlan& plan, hipStream_t s, int grid_limit, const Gemm
   HIP_CHECK(hipGetLastError());
 }
 
+// Small plans: a workgroup's eight waves split the k steps of a 16 x 16 tile
+// of outputs, or of two, four or eight of them next to each other where K is
+// short.  Bound by latency: a tile of the persistent
+// kernel walks K in chunks of 16, each a memory round trip and a barrier that
+// nothing else on the compute unit covers when there are few tiles, and the
+// tile shapes and row passes are separate launches.  Here every wave has all
+// operands of eight k steps (16 KB) in flight straight into MFMA operands, and
+// the partial sums meet in LDS once.  Without operand reuse it reads
+// 32 elements per k of a tile, from L2 while the plan is small.
+// Spin chain, chi=200: stages L and R 34 and 72 us in up to four launches each
+// -> 15 and 10 us, matvec 115 -> 32 us.
+constexpr int kDirectWaves = 8;
+
+// waves that share the k steps of a tile: eight steps each while there are
+// enough waves
+__host__ __device__ inline int direct_split(int64_t steps) {
+  return steps <= 8 ? 1 : steps <= 16 ? 2 : steps <= 32 ? 4 : kDirectWaves;
+}
+
+template <typename R>
+__global__ __launch_bounds__(64 * kDirectWaves) void direct_gemm_kernel(const GemmProb* __restrict__ probs,
+                                                                        const GemmSeg* __restrict__ segs,
+                                                                        const GemmTile* __restrict__ tiles, int ntiles,
+                                                                        GemmBases bases) {
+  using C = typename CT<R>::T;
+  using acc_t = typename Mf<R>::acc;
+  constexpr int U = 8;
+  __shared__ const C* sA[kDirectSegs];
+  __shared__ const C* sB[kDirectSegs];
+  __shared__ int64_t sLa[kDirectSegs], sLb[kDirectSegs];
+  __shared__ int sK[kDirectSegs], sStep[kDirectSegs + 1];
+  __shared__ C sum[kDirectWaves][256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fk = lane >> 4;
+  const int Gd = gridDim.x;
+  const int v0 = (Gd % kXcds == 0) ? (blockIdx.x % kXcds) * (Gd / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+  for (int t = v0; t < ntiles; t += Gd) {
+    const GemmTile tl = cload(tiles + t);
+    const GemmProb P = cload(probs + tl.prob);
+    if (t != v0) __syncthreads();              // the previous tile's tables and sums are no longer read
+    if (tid < 64) {
+      int k = 0;
+      if (tid < P.nseg) {
+        const GemmSeg S = segs[P.seg0 + tid];
+        const int asp = (S.flags >> 8) & 15, bsp = (S.flags >> 12) & 15;
+        sA[tid] = (asp ? reinterpret_cast<const C*>(bases.p[asp]) + reinterpret_cast<intptr_t>(S.A)
+                       : reinterpret_cast<const C*>(S.A)) +
+                  static_cast<int64_t>(tl.batch) * S.bsA;
+        sB[tid] = (bsp ? reinterpret_cast<const C*>(bases.p[bsp]) + reinterpret_cast<intptr_t>(S.B)
+                       : reinterpret_cast<const C*>(S.B)) +
+                  static_cast<int64_t>(tl.batch) * S.bsB;
+        sLa[tid] = S.csA;
+        sLb[tid] = S.ldB;
+        sK[tid] = k = S.K;
+      }
+      int st = (k + 3) / 4;                    // inclusive scan of the segments' k steps
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(st, o, 64);
+        if (lane >= o) st += v;
+      }
+      sStep[tid + 1] = st;
+      if (tid == 0) sStep[0] = 0;
+    }
+    const int32_t lay = P.nseg ? cload(segs + P.seg0).flags : 0;
+    const bool akc = lay & kSegAKContig, bnc = lay & kSegBNContig;
+    __syncthreads();
+    const int total = P.nseg ? sStep[P.nseg] : 0;
+    const int split = direct_split(total), share = wave % split;
+    const int nt = tl.n0 + wave / split * 16;  // this wave's tile
+    const int s_end = nt < P.N ? static_cast<int>(int64_t(total) * (share + 1) / split) : 0;
+    // rows and columns past the edge repeat the last one and are not stored
+    const int64_t m = min(tl.m0 + fr, P.M - 1), n = min(nt + fr, P.N - 1);
+    acc_t re{0, 0, 0, 0}, im{0, 0, 0, 0};
+    for (int s0 = static_cast<int>(int64_t(total) * share / split); s0 < s_end; s0 += U) {
+      // lane u finds the segment of step s0 + u
+      const int mine = min(s0 + (lane & (U - 1)), s_end - 1);
+      int lo = 0, hi = P.nseg - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (sStep[mid] <= mine) lo = mid;
+        else hi = mid - 1;
+      }
+      const int kk = (mine - sStep[lo]) * 4;
+      C a[U], b[U];
+      bool in[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = __builtin_amdgcn_readlane(lo, u);
+        const int k0 = __builtin_amdgcn_readlane(kk, u) + fk, K = sK[j];
+        const int64_t k = min(k0, K - 1);
+        in[u] = k0 < K && s0 + u < s_end;
+        a[u] = gload(sA[j] + (akc ? k + m * sLa[j] : m + k * sLa[j]));
+        b[u] = gload(sB[j] + (bnc ? n + k * sLb[j] : k + n * sLb[j]));
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const R ar = in[u] ? a[u].x : R(0), br = in[u] ? b[u].x : R(0);
+        R ai = in[u] ? a[u].y : R(0), bi = in[u] ? b[u].y : R(0);
+        if (lay & kSegConjA) ai = -ai;
+        if (lay & kSegConjB) bi = -bi;
+        re = Mf<R>::mma(br, ar, re);
+        im = Mf<R>::mma(br, ai, im);
+        re = Mf<R>::mma(-bi, ai, re);
+        im = Mf<R>::mma(bi, ar, im);
+      }
+    }
+    // element v of a lane is column row(fk, v), row fr
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      C c;
+      c.x = re[v];
+      c.y = im[v];
+      sum[wave][Mf<R>::row(fk, v) * 16 + fr] = c;
+    }
+    __syncthreads();
+    for (int e = tid; e < 256 * (kDirectWaves / split); e += 64 * kDirectWaves) {
+      const int g = e >> 8, o = e & 255;
+      const int mm = tl.m0 + (o & 15), nn = tl.n0 + g * 16 + (o >> 4);
+      if (mm >= P.M || nn >= P.N) continue;
+      C c = sum[g * split][o];
+      for (int w = 1; w < split; ++w) {
+        c.x += sum[g * split + w][o].x;
+        c.y += sum[g * split + w][o].y;
+      }
+      C* dst = (P.cspace ? reinterpret_cast<C*>(const_cast<void*>(bases.p[P.cspace])) + reinterpret_cast<intptr_t>(P.C)
+                         : reinterpret_cast<C*>(P.C)) +
+               (static_cast<int64_t>(tl.batch) * P.bsC + mm + static_cast<int64_t>(nn) * P.csC);
+      if (P.beta) {
+        const C old = gload(dst);
+        c.x += old.x;
+        c.y += old.y;
+      }
+      gstore(dst, c);
+    }
+  }
+}
+
+template <typename R>
+void launch_direct(const GemmPlan& plan, hipStream_t s, int grid_limit, const GemmBases& bases) {
+  const int n = static_cast<int>(plan.direct.size());
+  static int cus = device_cu_count();
+  int grid = std::min(n, cus * 4);
+  if (grid_limit > 0) grid = std::min(grid, grid_limit);
+  hipLaunchKernelGGL((direct_gemm_kernel<R>), dim3(grid), dim3(64 * kDirectWaves), 0, s, plan.d_probs.get(),
+                     plan.d_segs.get(), plan.d_direct.get(), n, bases);
+  HIP_CHECK(hipGetLastError());
+}
+
 template <typename R, int TM, int TN>
 void launch_shape(const GemmPlan& plan, const LaunchCfg& c, int shape, hipStream_t s, int grid_limit,
                   const GemmBases& bases) {
@@ -729,11 +878,6 @@ void GemmPlan::choose_tiles(int mode) {
   cfg[0].tile_mode = cfg[1].tile_mode = mode;
 }
 
-void GemmPlan::build_tiles() {
-  build_tiles_mode(cfg[0].tile_mode);
-  if (cfg[1].tile_mode != cfg[0].tile_mode) build_tiles_mode(cfg[1].tile_mode);
-}
-
 // Row pass or tiles: N <= 16 and K <= 32 per segment (see GemmPlan::rows).
 // Below the line the tiles lose: U(1) chi=1024 W stages 15.4 ms against 3.6,
 // spin chain chi=200 W stages 50 us against 9, chain d=64 chi=32 stage R 0.128
@@ -756,6 +900,93 @@ static bool row_eligible(const GemmPlan& plan, const GemmProb& p) {
     k += g.K;
   }
   return k <= kRowIn;
+}
+
+// tile shape of a problem under a policy
+static int tile_shape(const GemmProb& p, int mode) {
+  int shape = 0;
+  if (mode == 0) return shape;
+  double best = 1e300;
+  const int t_end = mode == 3 ? kNumTileShapes : kNumSmallShapes;
+  for (int t = (mode == 2 ? 1 : 0); t < t_end; ++t) {
+    const double tm = kTileShapes[t].tm, tn = kTileShapes[t].tn;
+    const double pm = std::ceil(p.M / tm) * tm, pn = std::ceil(p.N / tn) * tn;
+    // padded area, with a small per-tile overhead so bigger tiles win ties
+    const double c = pm * pn * (1.0 + 0.02 * (4096.0 / (tm * tn)));
+    if (c < best) { best = c; shape = t; }
+  }
+  return shape;
+}
+
+// Small plan, or tiles and row passes: whichever the latencies measured on
+// small spin and coupled chains make shorter (microseconds).  A tile launch
+// takes 5 and 1.4 per chunk of its longest K, a row pass 5; the direct kernel 7
+// for the first 1024 work items (what the chip holds) and 4 for every further
+// 1024, 2 per eight k steps of its longest wave, and 0.2 per 1000 k steps of all
+// tiles (operands from L2); a tenth must be gained.  Stage L / R of the spin chain, tiles against
+// direct: chi=50 10.6 / 13.0 and 10.7 / 13.1, 100 14.5 / 25.0 and 9.2 / 9.7, 200
+// 34.3 / 71.7 and 15.4 / 10.2, 400 57 / 139 and 41 / 26, 800 114 / 213 and 186 /
+// 150; 8-level chain chi=24 7.9 and 10.5 (L), 64 14.0 and 11.7 (R); 8-level U(1)
+// chain chi=64 (thousands of tiny problems) 14 and 48 (L).
+bool GemmPlan::build_direct() {
+  direct.clear();
+  direct_uploaded = false;
+  static const bool off = [] {
+    const char* e = std::getenv("CAM_DIRECT");
+    return e && *e == '0';
+  }();
+  if (off) return false;
+  auto steps_of = [&](const GemmProb& p) {
+    int64_t st = 0;
+    for (int q = p.seg0; q < p.seg0 + p.nseg; ++q) st += (segs[q].K + 3) / 4;
+    return st;
+  };
+  int64_t items = 0, steps = 0, wave_steps = 0, chunks[kNumTileShapes];
+  std::fill(std::begin(chunks), std::end(chunks), int64_t(-1));
+  bool rows_any = false, tiles_any = false;
+  for (const GemmProb& p : probs) {
+    if (p.M <= 0 || p.N <= 0 || p.batch <= 0) continue;
+    if (p.nseg > kDirectSegs) return false;
+    const int64_t st = steps_of(p);
+    const int split = direct_split(st), tn = 16 * (kDirectWaves / split);
+    const int64_t tm = (p.M + 15) / 16;
+    items += p.batch * tm * ((p.N + tn - 1) / tn);
+    steps += p.batch * tm * ((p.N + 15) / 16) * st;
+    wave_steps = std::max(wave_steps, (st + split - 1) / split);
+    if (row_eligible(*this, p)) {
+      rows_any = true;
+    } else {
+      tiles_any = true;
+      int64_t& c = chunks[tile_shape(p, 1)];
+      int64_t n = 0;
+      for (int q = p.seg0; q < p.seg0 + p.nseg; ++q) n += (segs[q].K + KCmax - 1) / KCmax;
+      c = std::max(c, n);
+    }
+    if (items > (1 << 16)) return false;
+  }
+  if (!tiles_any) return false;
+  double tiled = rows_any ? 5.0 : 0.0;
+  for (int64_t c : chunks)
+    if (c >= 0) tiled += 5.0 + 1.4 * static_cast<double>(c);
+  const double one = 7.0 + 4.0 * static_cast<double>((items - 1) / 1024) + 2.0 * static_cast<double>((wave_steps + 7) / 8) +
+                     2e-4 * static_cast<double>(steps);
+  if (1.1 * one >= tiled) return false;
+  direct.reserve(static_cast<size_t>(items));
+  for (size_t pi = 0; pi < probs.size(); ++pi) {
+    const GemmProb& p = probs[pi];
+    if (!p.nseg && p.beta) continue;   // nothing to add
+    const int tn = 16 * (kDirectWaves / direct_split(steps_of(p)));
+    for (int b = 0; b < p.batch; ++b)
+      for (int n0 = 0; n0 < p.N; n0 += tn)
+        for (int m0 = 0; m0 < p.M; m0 += 16) direct.push_back(GemmTile{static_cast<int32_t>(pi), b, m0, n0});
+  }
+  return !direct.empty();
+}
+
+void GemmPlan::build_tiles() {
+  if (build_direct()) return;
+  build_tiles_mode(cfg[0].tile_mode);
+  if (cfg[1].tile_mode != cfg[0].tile_mode) build_tiles_mode(cfg[1].tile_mode);
 }
 
 // Passes: problems with the same rows and the same input columns, up to
@@ -868,18 +1099,7 @@ void GemmPlan::build_tiles_mode(int mode) {
       row_probs.push_back(static_cast<int>(pi));
       continue;
     }
-    int shape = 0;
-    if (mode != 0) {
-      double best = 1e300;
-      const int t_end = mode == 3 ? kNumTileShapes : kNumSmallShapes;
-      for (int t = (mode == 2 ? 1 : 0); t < t_end; ++t) {
-        const double tm = kTileShapes[t].tm, tn = kTileShapes[t].tn;
-        const double pm = std::ceil(p.M / tm) * tm, pn = std::ceil(p.N / tn) * tn;
-        // padded area, with a small per-tile overhead so bigger tiles win ties
-        const double c = pm * pn * (1.0 + 0.02 * (4096.0 / (tm * tn)));
-        if (c < best) { best = c; shape = t; }
-      }
-    }
+    const int shape = tile_shape(p, mode);
     int64_t ktot = 0;
     for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) ktot += (segs[s].K + KCmax - 1) / KCmax * KCmax;
     if (ktot == 0 && p.beta) continue;   // nothing to add
@@ -951,6 +1171,10 @@ void GemmPlan::upload(hipStream_t s) {
     d_segs.upload(segs.data(), segs.size(), s);
     uploaded = true;
   }
+  if (!direct_uploaded) {
+    if (!direct.empty()) d_direct.upload(direct, s);
+    direct_uploaded = true;
+  }
   if (!rows_uploaded) {
     if (!rows.empty()) {
       static_assert(sizeof(RowIn) % 8 == 0 && sizeof(RowOut) % 8 == 0 && sizeof(RowBlk) % 8 == 0,
@@ -990,6 +1214,8 @@ void GemmPlan::clear() {
   row_blk.clear();
   rows.clear();
   rows_uploaded = false;
+  direct.clear();
+  direct_uploaded = false;
   for (int m = 0; m < kTileModes; ++m) {
     for (auto& t : tiles[m]) t.clear();
     built[m] = false;
@@ -1069,6 +1295,7 @@ bool autotune(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bas
     }
     return best;
   };
+  // (a plan large enough to be tuned is never a small one)
   // coordinate descent: product form, then tile policy, then K chunk, then
   // grid size
   LaunchCfg cur = plan.cfg[precision];
@@ -1103,6 +1330,14 @@ bool autotune(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bas
 void launch_grouped_gemm(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bases,
                          int grid_limit) {
   const LaunchCfg& c = plan.cfg[precision];
+  if (c.direct && !plan.direct.empty()) {
+    if (!plan.uploaded || !plan.direct_uploaded) plan.upload(s);
+    GemmBases b{};
+    if (bases) b = *bases;
+    if (precision == 0) launch_direct<double>(plan, s, grid_limit, b);
+    else launch_direct<float>(plan, s, grid_limit, b);
+    return;
+  }
   if (!plan.built[c.tile_mode]) plan.build_tiles_mode(c.tile_mode);
   if (!plan.uploaded || !plan.tiles_uploaded[c.tile_mode]) plan.upload(s);
   GemmBases b{};

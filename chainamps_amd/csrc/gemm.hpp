@@ -97,6 +97,8 @@ struct RowItem {                // rows [.., + rows) of a pass, from row m0 of b
   int32_t conjA, beta;
 };
 
+constexpr int kDirectSegs = 64;    // segments of one problem of a small plan (see GemmPlan::direct)
+
 // Tile shapes compiled into the kernels (TM x TN per workgroup).
 struct TileShape { int tm, tn; };
 constexpr int kNumTileShapes = 6;
@@ -118,6 +120,7 @@ struct LaunchCfg {
                         //    (fewer operand re-reads per flop)
   int wg_per_cu = 4;    // persistent grid = min(tiles, CUs * wg_per_cu)
   int kc = 16;          // K chunk per LDS stage: 16 or 8 (half the LDS)
+  bool direct = true;   // small plans take the one-launch kernel (false: tiles)
 };
 
 struct GemmPlan {
@@ -145,6 +148,11 @@ struct GemmPlan {
   int row_lds = 0;                        // largest padded matrix (elements)
   DevBuf<int64_t> d_rows;                 // all four, in the order in, out, blocks, items
   bool rows_uploaded = false;
+  // Plans too small to fill the chip with tiles: one launch for all problems,
+  // a workgroup per 16 x 16 outputs (empty: tiles and row passes).
+  std::vector<GemmTile> direct;
+  DevBuf<GemmTile> d_direct;
+  bool direct_uploaded = false;
   // Per problem, a row group (-1: none).  Problems of one group read the
   // same A rows (one output per MPO channel from the same operand rows), so
   // their tiles of equal (batch, m0) are ordered next to each other and run
@@ -158,9 +166,11 @@ struct GemmPlan {
   void set_group(int prob, int64_t g);
   // tile-shape policy for both precisions (see LaunchCfg::tile_mode)
   void choose_tiles(int mode);
-  // tiles of the selected policies, LPT-sorted
+  // a small plan's list, or the tiles of the selected policies, LPT-sorted
   void build_tiles();
   void build_tiles_mode(int mode);
+  // the list of a small plan; false for any other
+  bool build_direct();
   // tables and items of the row passes over the given problems
   void build_rows(const std::vector<int>& eligible);
   // Histogram signature: problems bucketed by (log2 M, log2 N, log2 K,
