@@ -1205,6 +1205,12 @@ void GemmPlan::upload(hipStream_t s) {
   }
 }
 
+bool GemmPlan::on_device(int precision) const {
+  const LaunchCfg& c = cfg[precision];
+  if (c.direct && !direct.empty()) return uploaded && direct_uploaded;
+  return uploaded && rows_uploaded && built[c.tile_mode] && tiles_uploaded[c.tile_mode];
+}
+
 void GemmPlan::clear() {
   probs.clear();
   segs.clear();
@@ -1331,7 +1337,7 @@ void launch_grouped_gemm(GemmPlan& plan, int precision, hipStream_t s, const Gem
                          int grid_limit) {
   const LaunchCfg& c = plan.cfg[precision];
   if (c.direct && !plan.direct.empty()) {
-    if (!plan.uploaded || !plan.direct_uploaded) plan.upload(s);
+    if (!plan.on_device(precision)) plan.upload(s);
     GemmBases b{};
     if (bases) b = *bases;
     if (precision == 0) launch_direct<double>(plan, s, grid_limit, b);
@@ -1339,7 +1345,7 @@ void launch_grouped_gemm(GemmPlan& plan, int precision, hipStream_t s, const Gem
     return;
   }
   if (!plan.built[c.tile_mode]) plan.build_tiles_mode(c.tile_mode);
-  if (!plan.uploaded || !plan.tiles_uploaded[c.tile_mode]) plan.upload(s);
+  if (!plan.on_device(precision)) plan.upload(s);
   GemmBases b{};
   if (bases) b = *bases;
   if (precision == 0) {

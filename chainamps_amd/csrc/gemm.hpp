@@ -178,6 +178,8 @@ struct GemmPlan {
   uint64_t signature(int precision) const;
   // problems, segments and every built tile list to the device
   void upload(hipStream_t s);
+  // whether a launch at this precision finds all it needs on the device
+  bool on_device(int precision) const;
   void clear();
 };
 

@@ -63,12 +63,10 @@ void heff_apply_noalloc(Heff& H, const cplx* in, cplx* out) {
   // the plans must already be on the device at their current launch
   // configuration: uploading them (or autotuning) would allocate
   for (const auto& st : H.plans)
-    for (const GemmPlan& p : st) {
-      const LaunchCfg& c = p.cfg[0];
-      CAM_REQUIRE(p.uploaded && p.built[c.tile_mode] && p.tiles_uploaded[c.tile_mode],
+    for (const GemmPlan& p : st)
+      CAM_REQUIRE(p.on_device(0),
                   "noalloc: the matvec plans are not on the device at their launch configuration "
                   "(run cam_heff_apply_blocked once, or cam_heff_set_launch, before this call)");
-    }
   hipStream_t s = H.ctx->stream;
   cplx* t1 = static_cast<cplx*>(base);
   cplx* t2 = t1 + H.ws1n;

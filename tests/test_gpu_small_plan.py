@@ -53,3 +53,20 @@ def test_sectors(ctx, chi):
     rng = np.random.default_rng(chi)
     v = rng.standard_normal(H.n) + 1j * rng.standard_normal(H.n)
     assert rel_err(H.apply(v), T.apply(v)) <= 1e-13
+
+
+def test_noalloc(ctx):
+    """The no-allocation matvec accepts a small plan that has not run yet."""
+    print("case small_plan noalloc", flush=True)
+    import chainamps_amd as cam
+    import torch
+    rng = np.random.default_rng(5)
+    _, ups = _env(rng, 100, 1, 4)
+    H = cam.Heff(*(u(ctx) for u in ups))
+    x = torch.from_numpy(_rand(rng, H.n)).cuda()
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    torch.cuda.synchronize()
+    H.apply_device_noalloc(x.data_ptr(), y.data_ptr())
+    H.apply_device(x.data_ptr(), z.data_ptr())
+    ctx.sync()
+    assert torch.equal(y, z)
