@@ -11,6 +11,7 @@ import pytest
 
 from conftest import rel_err
 from test_gpu_gemm_edges import _env, _rand
+from test_zz_no_alloc import DevVec, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -59,14 +60,17 @@ def test_noalloc(ctx):
     """The no-allocation matvec accepts a small plan that has not run yet."""
     print("case small_plan noalloc", flush=True)
     import chainamps_amd as cam
-    import torch
+    hip = _hip()
     rng = np.random.default_rng(5)
     _, ups = _env(rng, 100, 1, 4)
     H = cam.Heff(*(u(ctx) for u in ups))
-    x = torch.from_numpy(_rand(rng, H.n)).cuda()
-    y, z = torch.empty_like(x), torch.empty_like(x)
-    torch.cuda.synchronize()
-    H.apply_device_noalloc(x.data_ptr(), y.data_ptr())
-    H.apply_device(x.data_ptr(), z.data_ptr())
-    ctx.sync()
-    assert torch.equal(y, z)
+    x, y, z = (DevVec(hip, H.n) for _ in range(3))
+    try:
+        x.upload(_rand(rng, H.n))
+        H.apply_device_noalloc(x.ptr, y.ptr)
+        H.apply_device(x.ptr, z.ptr)
+        ctx.sync()
+        assert np.array_equal(y.download(), z.download())
+    finally:
+        for b in (x, y, z):
+            b.free()
