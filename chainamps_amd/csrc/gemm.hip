@@ -20,6 +20,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -625,11 +626,8 @@ void launch_rows(const GemmPlan& plan, hipStream_t s, int grid_limit, const Gemm
   int grid = std::min(n, cus * 8);
   if (grid_limit > 0) grid = std::min(grid, grid_limit);
   const size_t lds = static_cast<size_t>(plan.row_lds) * sizeof(typename CT<R>::T);
-  const RowIn* in = reinterpret_cast<const RowIn*>(plan.d_rows.get());
-  const RowOut* out = reinterpret_cast<const RowOut*>(in + plan.row_in.size());
-  const RowBlk* blk = reinterpret_cast<const RowBlk*>(out + plan.row_out.size());
-  const RowItem* items = reinterpret_cast<const RowItem*>(blk + plan.row_blk.size());
-  hipLaunchKernelGGL((row_gemm_kernel<R>), dim3(grid), dim3(kRowThreads), lds, s, items, n, in, out, blk, bases);
+  hipLaunchKernelGGL((row_gemm_kernel<R>), dim3(grid), dim3(kRowThreads), lds, s, plan.d_rows, n, plan.d_row_in,
+                     plan.d_row_out, plan.d_row_blk, bases);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -777,8 +775,8 @@ void launch_direct(const GemmPlan& plan, hipStream_t s, int grid_limit, const Ge
   static int cus = device_cu_count();
   int grid = std::min(n, cus * 4);
   if (grid_limit > 0) grid = std::min(grid, grid_limit);
-  hipLaunchKernelGGL((direct_gemm_kernel<R>), dim3(grid), dim3(64 * kDirectWaves), 0, s, plan.d_probs.get(),
-                     plan.d_segs.get(), plan.d_direct.get(), n, bases);
+  hipLaunchKernelGGL((direct_gemm_kernel<R>), dim3(grid), dim3(64 * kDirectWaves), 0, s, plan.d_probs,
+                     plan.d_segs, plan.d_direct, n, bases);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -790,9 +788,9 @@ void launch_shape(const GemmPlan& plan, const LaunchCfg& c, int shape, hipStream
   static int cus = device_cu_count();
   int grid = std::min(nt, cus * std::max(1, c.wg_per_cu));
   if (grid_limit > 0) grid = std::min(grid, grid_limit);
-  const GemmTile* tiles = plan.d_tiles[c.tile_mode][shape].get();
-  const GemmProb* P = plan.d_probs.get();
-  const GemmSeg* S = plan.d_segs.get();
+  const GemmTile* tiles = plan.d_tiles[c.tile_mode][shape];
+  const GemmProb* P = plan.d_probs;
+  const GemmSeg* S = plan.d_segs;
   auto go = [&](auto g3, auto kc) {
     hipLaunchKernelGGL((grouped_gemm_kernel<R, TM, TN, decltype(g3)::value, decltype(kc)::value>), dim3(grid),
                        dim3(Waves<R, TM, TN>::kThreads), 0, s, P, S, tiles, nt, bases);
@@ -830,7 +828,7 @@ int GemmPlan::add_problem(void* C, int64_t csC, int M, int N, int batch, int64_t
   p.cspace = cspace;
   probs.push_back(p);
   group.push_back(-1);
-  uploaded = false;
+  uploaded = rows_built = false;
   for (int m = 0; m < kTileModes; ++m) built[m] = tiles_uploaded[m] = false;
   return static_cast<int>(probs.size()) - 1;
 }
@@ -838,6 +836,7 @@ int GemmPlan::add_problem(void* C, int64_t csC, int M, int N, int batch, int64_t
 void GemmPlan::set_group(int prob, int64_t g) {
   CAM_REQUIRE(prob >= 0 && prob < static_cast<int>(probs.size()), "set_group: no such problem");
   group[prob] = g;
+  rows_built = false;
   for (int m = 0; m < kTileModes; ++m) built[m] = tiles_uploaded[m] = false;
 }
 
@@ -870,7 +869,7 @@ void GemmPlan::add_segment(int prob, const void* A, int64_t csA, int64_t bsA, co
   segs.push_back(g);
   p.nseg++;
   flops += 8.0 * double(p.M) * double(p.N) * double(K) * double(p.batch);
-  uploaded = false;
+  uploaded = rows_built = false;
 }
 
 void GemmPlan::choose_tiles(int mode) {
@@ -999,6 +998,7 @@ void GemmPlan::build_rows(const std::vector<int>& eligible) {
   row_blk.clear();
   rows.clear();
   row_lds = 0;
+  rows_built = true;
   rows_uploaded = false;
   if (eligible.empty()) return;
   struct Pass { std::vector<int> probs; int nout = 0; };
@@ -1158,51 +1158,53 @@ void GemmPlan::build_tiles_mode(int mode) {
     for (auto o : ord) sorted.push_back(T[t][o]);
     T[t].swap(sorted);
   }
-  build_rows(row_probs);
+  if (!rows_built) build_rows(row_probs);   // the same for every policy
   built[mode] = true;
   tiles_uploaded[mode] = false;
 }
 
 void GemmPlan::upload(hipStream_t s) {
   if (!uploaded) {
-    d_probs.ensure(std::max<size_t>(probs.size(), 1));
-    d_probs.upload(probs.data(), probs.size(), s);
-    d_segs.ensure(std::max<size_t>(segs.size(), 1));
-    d_segs.upload(segs.data(), segs.size(), s);
-    uploaded = true;
+    // a new set of problems: nothing on the device holds any more (freeing
+    // waits for launches that still read it)
+    d_bufs.clear();
+    rows_uploaded = direct_uploaded = false;
+    for (int m = 0; m < kTileModes; ++m) tiles_uploaded[m] = false;
   }
-  if (!direct_uploaded) {
-    if (!direct.empty()) d_direct.upload(direct, s);
-    direct_uploaded = true;
+  std::vector<char> host;
+  std::vector<std::function<void(const char*)>> placed;
+  auto put = [&](const auto& v, auto& d) {
+    d = nullptr;
+    if (v.empty()) return;
+    const size_t at = (host.size() + 15) / 16 * 16;
+    host.resize(at + v.size() * sizeof(v[0]));
+    std::memcpy(host.data() + at, v.data(), v.size() * sizeof(v[0]));
+    placed.emplace_back([&d, at](const char* base) {
+      d = reinterpret_cast<std::remove_reference_t<decltype(d)>>(base + at);
+    });
+  };
+  if (!uploaded) {
+    put(probs, d_probs);
+    put(segs, d_segs);
   }
+  if (!direct_uploaded) put(direct, d_direct);
   if (!rows_uploaded) {
-    if (!rows.empty()) {
-      static_assert(sizeof(RowIn) % 8 == 0 && sizeof(RowOut) % 8 == 0 && sizeof(RowBlk) % 8 == 0,
-                    "the row tables lie one after another");
-      auto words = [](size_t bytes) { return (bytes + 7) / 8; };
-      std::vector<int64_t> h(words(row_in.size() * sizeof(RowIn) + row_out.size() * sizeof(RowOut) +
-                                   row_blk.size() * sizeof(RowBlk) + rows.size() * sizeof(RowItem)));
-      char* q = reinterpret_cast<char*>(h.data());
-      auto put = [&q](const auto& v) {
-        std::memcpy(q, v.data(), v.size() * sizeof(v[0]));
-        q += v.size() * sizeof(v[0]);
-      };
-      put(row_in);
-      put(row_out);
-      put(row_blk);
-      put(rows);
-      d_rows.upload(h, s);
-    }
-    rows_uploaded = true;
+    put(row_in, d_row_in);
+    put(row_out, d_row_out);
+    put(row_blk, d_row_blk);
+    put(rows, d_rows);
   }
-  for (int m = 0; m < kTileModes; ++m) {
-    if (!built[m] || tiles_uploaded[m]) continue;
-    for (int t = 0; t < kNumTileShapes; ++t) {
-      d_tiles[m][t].ensure(std::max<size_t>(tiles[m][t].size(), 1));
-      d_tiles[m][t].upload(tiles[m][t].data(), tiles[m][t].size(), s);
-    }
-    tiles_uploaded[m] = true;
+  for (int m = 0; m < kTileModes; ++m)
+    if (built[m] && !tiles_uploaded[m])
+      for (int t = 0; t < kNumTileShapes; ++t) put(tiles[m][t], d_tiles[m][t]);
+  if (!host.empty()) {
+    DevBuf<char> buf(host.size());
+    buf.upload(host.data(), host.size(), s);
+    for (auto& set : placed) set(buf.get());
+    d_bufs.push_back(std::move(buf));
   }
+  uploaded = direct_uploaded = rows_uploaded = true;
+  for (int m = 0; m < kTileModes; ++m) tiles_uploaded[m] = built[m];
 }
 
 bool GemmPlan::on_device(int precision) const {
@@ -1219,7 +1221,7 @@ void GemmPlan::clear() {
   row_out.clear();
   row_blk.clear();
   rows.clear();
-  rows_uploaded = false;
+  rows_built = rows_uploaded = false;
   direct.clear();
   direct_uploaded = false;
   for (int m = 0; m < kTileModes; ++m) {

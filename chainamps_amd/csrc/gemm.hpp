@@ -128,9 +128,14 @@ struct GemmPlan {
   std::vector<GemmSeg> segs;
   std::vector<GemmTile> tiles[kTileModes][kNumTileShapes];
   double flops = 0.0;          // algorithmic 8*m*n*k
-  DevBuf<GemmProb> d_probs;
-  DevBuf<GemmSeg> d_segs;
-  DevBuf<GemmTile> d_tiles[kTileModes][kNumTileShapes];
+  // Device copies.  Whatever an upload finds missing goes up in one buffer
+  // and one copy (a plan of a small tensor contraction lives for one launch,
+  // and an allocation, a free and a copy cost some 1, 1 and 4 us: growth run of
+  // the spin chain to chi=48 21.9 -> 20.1 ms, iTEBD to chi=32 7.8 -> 7.2).
+  std::vector<DevBuf<char>> d_bufs;
+  const GemmProb* d_probs = nullptr;
+  const GemmSeg* d_segs = nullptr;
+  const GemmTile* d_tiles[kTileModes][kNumTileShapes] = {};
   bool uploaded = false;                  // problems and segments
   bool built[kTileModes] = {false, false, false};
   bool tiles_uploaded[kTileModes] = {false, false, false};
@@ -146,12 +151,15 @@ struct GemmPlan {
   std::vector<RowBlk> row_blk;
   std::vector<RowItem> rows;
   int row_lds = 0;                        // largest padded matrix (elements)
-  DevBuf<int64_t> d_rows;                 // all four, in the order in, out, blocks, items
-  bool rows_uploaded = false;
+  const RowIn* d_row_in = nullptr;
+  const RowOut* d_row_out = nullptr;
+  const RowBlk* d_row_blk = nullptr;
+  const RowItem* d_rows = nullptr;
+  bool rows_built = false, rows_uploaded = false;
   // Plans too small to fill the chip with tiles: one launch for all problems,
   // a workgroup per 16 x 16 outputs (empty: tiles and row passes).
   std::vector<GemmTile> direct;
-  DevBuf<GemmTile> d_direct;
+  const GemmTile* d_direct = nullptr;
   bool direct_uploaded = false;
   // Per problem, a row group (-1: none).  Problems of one group read the
   // same A rows (one output per MPO channel from the same operand rows), so
