@@ -139,7 +139,12 @@ struct GemmPlan {
   bool uploaded = false;                  // problems and segments
   bool built[kTileModes] = {false, false, false};
   bool tiles_uploaded[kTileModes] = {false, false, false};
-  LaunchCfg cfg[2];                       // per precision (0 FP64, 1 FP32)
+  // Per precision (0 FP64, 1 FP32); plans below the tuning threshold keep the
+  // defaults.  FP64 starts from chunks of 8 (more workgroups resident; stages
+  // L, B, C, R with 16 and 8, us: chain d=64 chi=64 189 253 259 255 and 166 230
+  // 233 241, chi=32 58 59 59 35 and 48 54 54 36, U(1) d=20 chi=300 L / R 164 218
+  // and 131 194); in FP32 the two are level (107 138 143 139, 105 144 145 143).
+  LaunchCfg cfg[2] = {{kAlgo3M, 1, 4, 8, true}, {}};
   bool tuned[2] = {false, false};
   // Problems with at most kRowN columns whose segments all have K <= kRowK
   // and an M-contiguous A (W stages and environments of small QN sectors: a
