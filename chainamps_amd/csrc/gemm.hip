@@ -1003,27 +1003,42 @@ void GemmPlan::build_rows(const std::vector<int>& eligible) {
   if (eligible.empty()) return;
   struct Pass { std::vector<int> probs; int nout = 0; };
   std::vector<Pass> passes;
-  std::map<std::vector<int64_t>, int> open;   // input signature -> pass still being filled
+  constexpr int32_t kPerProblem = kSegConjB | kSegBNContig;   // B's layout may differ within a pass
+  auto same_inputs = [&](const GemmProb& x, const GemmProb& y) {
+    if (x.M != y.M || x.batch != y.batch || x.beta != y.beta || x.cspace != y.cspace || x.nseg != y.nseg) return false;
+    for (int j = 0; j < x.nseg; ++j) {
+      const GemmSeg &f = segs[x.seg0 + j], &g = segs[y.seg0 + j];
+      if (f.A != g.A || f.csA != g.csA || f.bsA != g.bsA || f.K != g.K || ((f.flags ^ g.flags) & ~kPerProblem))
+        return false;
+    }
+    return true;
+  };
+  std::unordered_multimap<uint64_t, int> open;   // hash of the inputs -> pass still being filled
+  open.reserve(eligible.size());
   for (int pi : eligible) {
     const GemmProb& p = probs[pi];
-    std::vector<int64_t> key{p.M, p.batch, p.beta, p.cspace};
+    uint64_t h = 1469598103934665603ull;
+    auto mix = [&h](uint64_t v) { h = (h ^ v) * 1099511628211ull; };
+    mix(static_cast<uint64_t>(p.M));
+    mix(static_cast<uint64_t>(p.batch));
     int nin = 0;
     for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) {
-      const GemmSeg& g = segs[s];
-      key.insert(key.end(), {reinterpret_cast<int64_t>(g.A), g.csA, g.bsA, g.K,
-                             g.flags & ~(kSegConjB | kSegBNContig)});
-      nin += g.K;
+      mix(reinterpret_cast<uint64_t>(segs[s].A));
+      nin += segs[s].K;
     }
     const int kp = (nin + 3) / 4 * 4;
-    auto it = open.find(key);
-    if (it != open.end()) {
-      const int no = passes[it->second].nout + p.N;
-      if (no > kRowOut || kp * ((no + 15) / 16 * 16) > kRowB) it = open.end();
-    }
-    if (it == open.end()) {
-      open[key] = static_cast<int>(passes.size());
+    const auto range = open.equal_range(h);
+    auto it = range.first;
+    while (it != range.second && !same_inputs(p, probs[passes[it->second].probs[0]])) ++it;
+    if (it == range.second) {
+      it = open.emplace(h, static_cast<int>(passes.size()));
       passes.emplace_back();
-      it = open.find(key);
+    } else {
+      const int no = passes[it->second].nout + p.N;
+      if (no > kRowOut || kp * ((no + 15) / 16 * 16) > kRowB) {
+        it->second = static_cast<int>(passes.size());
+        passes.emplace_back();
+      }
     }
     passes[it->second].probs.push_back(pi);
     passes[it->second].nout += p.N;
@@ -1034,8 +1049,7 @@ void GemmPlan::build_rows(const std::vector<int>& eligible) {
   for (const Pass& q : passes) total += int64_t(probs[q.probs[0]].M) * probs[q.probs[0]].batch;
   int per = 1024;
   while (per > 16 * kRowWaves && total / per < 2048) per /= 2;
-  struct Key { int64_t g, r0; int pass; };
-  std::vector<std::pair<Key, RowItem>> items;
+  std::vector<RowItem> first(passes.size());     // a pass's tables, without rows
   for (size_t qi = 0; qi < passes.size(); ++qi) {
     const Pass& q = passes[qi];
     const GemmProb& p0 = probs[q.probs[0]];
@@ -1068,24 +1082,36 @@ void GemmPlan::build_rows(const std::vector<int>& eligible) {
     it.conjA = (g0.flags & kSegConjA) ? 1 : 0;
     it.beta = p0.beta;
     row_lds = std::max(row_lds, (it.nin + 3) / 4 * 4 * ((it.nout + 15) / 16 * 16));
-    const int64_t all = int64_t(p0.M) * p0.batch;
-    const int64_t g = group[q.probs[0]] >= 0 ? group[q.probs[0]] : -1 - q.probs[0];
-    for (int64_t r0 = 0; r0 < all; r0 += per) {
-      it.batch0 = static_cast<int32_t>(r0 / p0.M);
-      it.m0 = static_cast<int32_t>(r0 % p0.M);
-      it.rows = static_cast<int32_t>(std::min<int64_t>(per, all - r0));
-      items.push_back({Key{g, r0, static_cast<int>(qi)}, it});
-    }
+    first[qi] = it;
   }
   // passes of one row group next to each other at equal rows: they read the
   // same operand (from one XCD's L2 the second time)
-  std::stable_sort(items.begin(), items.end(), [](const auto& x, const auto& y) {
-    if (x.first.g != y.first.g) return x.first.g < y.first.g;
-    if (x.first.r0 != y.first.r0) return x.first.r0 < y.first.r0;
-    return x.first.pass < y.first.pass;
-  });
-  rows.reserve(items.size());
-  for (auto& e : items) rows.push_back(e.second);
+  auto group_of = [&](size_t qi) {
+    const int pi = passes[qi].probs[0];
+    return group[pi] >= 0 ? group[pi] : -1 - int64_t(pi);
+  };
+  std::vector<std::pair<int64_t, int>> order(passes.size());
+  for (size_t qi = 0; qi < passes.size(); ++qi) order[qi] = {group_of(qi), static_cast<int>(qi)};
+  std::sort(order.begin(), order.end());
+  for (size_t i0 = 0, i1; i0 < order.size(); i0 = i1) {
+    int64_t most = 0;
+    for (i1 = i0; i1 < order.size() && order[i1].first == order[i0].first; ++i1) {
+      const GemmProb& p = probs[passes[order[i1].second].probs[0]];
+      most = std::max(most, int64_t(p.M) * p.batch);
+    }
+    for (int64_t r0 = 0; r0 < most; r0 += per)
+      for (size_t i = i0; i < i1; ++i) {
+        const int qi = order[i].second;
+        const GemmProb& p = probs[passes[qi].probs[0]];
+        const int64_t all = int64_t(p.M) * p.batch;
+        if (r0 >= all) continue;
+        RowItem it = first[qi];
+        it.batch0 = static_cast<int32_t>(r0 / p.M);
+        it.m0 = static_cast<int32_t>(r0 % p.M);
+        it.rows = static_cast<int32_t>(std::min<int64_t>(per, all - r0));
+        rows.push_back(it);
+      }
+  }
 }
 
 void GemmPlan::build_tiles_mode(int mode) {
@@ -1172,6 +1198,8 @@ void GemmPlan::upload(hipStream_t s) {
     for (int m = 0; m < kTileModes; ++m) tiles_uploaded[m] = false;
   }
   std::vector<char> host;
+  host.reserve(probs.size() * sizeof(GemmProb) + segs.size() * sizeof(GemmSeg) + rows.size() * sizeof(RowItem) +
+               (row_in.size() + row_out.size()) * sizeof(RowIn) + row_blk.size() * sizeof(RowBlk) + 1024);
   std::vector<std::function<void(const char*)>> placed;
   auto put = [&](const auto& v, auto& d) {
     d = nullptr;
