@@ -118,6 +118,15 @@ __device__ __forceinline__ void rotate(const Rot& r, double2& x, double2& y) {
   y = r.swap ? u : v;
 }
 
+// Orders the LDS accesses of a wave's lanes where one lane reads what another
+// has just written: the hardware keeps a wave's LDS operations in order, this
+// keeps the compiler from moving them (no instruction of its own).
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // round-robin: pair k of round `step` among n (even) players
 __device__ __forceinline__ void round_robin(int n, int step, int k, int& lo, int& hi) {
   const int a = k == 0 ? n - 1 : (step + k) % (n - 1);
@@ -219,7 +228,8 @@ __device__ __forceinline__ void householder(double2* x, int j, int L, int l, dou
     x[j] = make_double2(ph.x * (aa + nx), ph.y * (aa + nx));
   }
 }
-// y <- (1 - tau v v^H) y over rows j.. (16 lanes)
+// y <- (1 - tau v v^H) y over rows j.. (16 lanes); the caller may go on with
+// rows of y that other lanes updated
 __device__ __forceinline__ void reflect(const double2* v, double tau, double2* y, int j, int L, int l) {
   double gr = 0, gi = 0;
   for (int r = j + l; r < L; r += 16) {
@@ -236,6 +246,7 @@ __device__ __forceinline__ void reflect(const double2* v, double tau, double2* y
     b.y -= gr * a.y + gi * a.x;
     y[r] = b;
   }
+  wave_order();
 }
 
 constexpr int kRowsPerLane = 9;   // rows per lane of a pair the sweeps are compiled for
@@ -835,6 +846,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(const QrJob* __res
         b.y -= g.x * a.y + g.y * a.x;
         y[r] = b;
       }
+      wave_order();
       if (wave == j + 1) make(j + 1);
     }
     __syncthreads();
@@ -860,9 +872,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(const QrJob* __res
           t.y -= tau[j] * p.y;
         }
       if (i == j) t.x = tau[j];
-      __builtin_amdgcn_wave_barrier();
+      wave_order();
       if (i <= j) T[i][j] = t;
-      __builtin_amdgcn_wave_barrier();
+      wave_order();
     }
   }
   __syncthreads();

@@ -67,3 +67,36 @@ def test_jacobi_rank_deficient(ctx, n, rank):
     _check(ctx, _rand(rng, n, rank) @ _rand(rng, rank, n))
     # exactly dependent columns: exact zeros appear during the rotations
     _check(ctx, np.tile(_rand(rng, n, 1), (1, n)) * np.where(np.arange(n) % 2, -1.0, 1.0))
+
+
+# On both sides of the switch from 16 to 8 columns per QR panel (more than 600
+# rows of the taller side), trailing columns that start off a multiple of 16,
+# and the largest columns and rows the kernels take.  The rounding grows like
+# the square root of the longer side: sqrt(1200 / 260) = 2.15 times the bounds
+# above, in the Frobenius norm.
+def _check_large(ctx, A):
+    U, s, Vd = _svd(ctx, A)
+    ref = np.linalg.svd(A, compute_uv=False)
+    k = len(ref)
+    assert len(s) == k
+    assert np.all(np.diff(s) <= 0)
+    assert np.abs(s - ref).max() <= 2.2e-13 * ref[0]
+    assert np.linalg.norm((U * s) @ Vd - A) <= 2.2e-13 * np.linalg.norm(A)
+    assert np.abs(U.conj().T @ U - np.eye(k)).max() <= 2.2e-12
+    assert np.abs(Vd @ Vd.conj().T - np.eye(k)).max() <= 2.2e-12
+
+
+@pytest.mark.parametrize("m,n", [(600, 70), (601, 70), (70, 601), (1200, 64), (90, 1200), (1200, 9), (640, 600),
+                                 (700, 650), (1000, 1024), (1024, 1024)])
+def test_jacobi_large(ctx, m, n):
+    print(f"case jacobi_large m={m} n={n}", flush=True)
+    rng = np.random.default_rng(1000 * m + n)
+    _check_large(ctx, _rand(rng, m, n))
+
+
+@pytest.mark.parametrize("m,n", [(640, 600), (70, 601), (1024, 1000)])
+def test_jacobi_large_rank_deficient(ctx, m, n):
+    print(f"case jacobi_large_rank_deficient m={m} n={n}", flush=True)
+    rng = np.random.default_rng(m + n)
+    _check_large(ctx, _rand(rng, m, 7) @ _rand(rng, 7, n))
+    _check_large(ctx, np.tile(_rand(rng, m, 1), (1, n)) * np.where(np.arange(n) % 2, -1.0, 1.0))
