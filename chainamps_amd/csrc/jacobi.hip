@@ -740,10 +740,10 @@ struct QrJob {
   double2* diag;         // R's diagonal
   double2* X;            // c x cp
   double2* V;            // c x cp
-  double2* Y;            // L x c: left vectors
+  double2* Y;            // L x ny: columns that Q is applied to (left vectors)
   double* len2;          // column lengths of A (A^H), squared
   int* perm;             // sorted position -> column
-  int m, n, L, c, cp, w, npan;
+  int m, n, L, c, cp, w, npan, ny;
   double scale;
 };
 
@@ -885,15 +885,15 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(const QrJob* __res
 }
 
 // Columns Y (16 per workgroup) <- (1 - V T' V^H) Y over rows j0.. of a panel:
-// T' = T^H on the trailing columns of B (onq = 0), T on the left vectors.
+// T' = T^H on the trailing columns of B (onq = 0), T on Y.
 // MFMA for V^H Y (rows split over the four waves) and for V (T' V^H Y).
 __global__ __launch_bounds__(256) void reflect_kernel(const QrJob* __restrict__ jobs, int pan, int onq) {
   __shared__ double2 red[4][kB][kB + 1], W[kB][kB + 1];
   const QrJob J = jobs[blockIdx.y];
   if (pan >= J.npan) return;
   const int j0 = pan * J.w, w = min(J.w, J.c - j0);
-  const int c0 = (onq ? 0 : j0 + w) + blockIdx.x * kB;
-  if (c0 >= J.c || (onq && !J.Y)) return;
+  const int c0 = (onq ? 0 : j0 + w) + blockIdx.x * kB, cols = onq ? J.ny : J.c;
+  if (c0 >= cols || (onq && !J.Y)) return;
   double2* const Y = onq ? J.Y : J.B;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int fr = lane & 15, fk = lane >> 4;
@@ -902,7 +902,7 @@ __global__ __launch_bounds__(256) void reflect_kernel(const QrJob* __restrict__ 
   auto vat = [&](int t, int64_t r) {
     return t < w && r >= j0 + t && r < L ? J.B[r + (j0 + t) * L] : make_double2(0.0, 0.0);
   };
-  const bool cin = c0 + fr < J.c;
+  const bool cin = c0 + fr < cols;
   {
     d4v re{0, 0, 0, 0}, im{0, 0, 0, 0};
     for (int64_t r0 = j0 + wave * 16; r0 < L; r0 += 64) {
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(256) void reflect_kernel(const QrJob* __restrict__ 
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int k = c0 + fk + 4 * v;
-        if (k < J.c) {
+        if (k < cols) {
           double2 y = Y[r + k * L];
           y.x -= re[v];
           y.y -= im[v];
@@ -1007,76 +1007,40 @@ __global__ __launch_bounds__(64) void norms_kernel(const QrJob* __restrict__ job
   }
 }
 
-// Null columns of X (rx = 0; elsewhere 1 / |x|) are replaced by unit vectors
-// completing the others, as in the LDS form; one workgroup per block.
+// Null columns of X (an exactly rank-deficient block) are replaced by unit
+// vectors that complete the others: with the r others, normalised, as B = Q R,
+// the last c - r columns of Q.  On the panel kernels this takes about what the
+// block's own QR does; unit vectors projected off every column one after
+// another by one workgroup took 788 ms of the 798 ms of a 1024-column block of
+// rank one (zgesvd: 328 ms).
 struct NullJob {
-  double2* X;
-  double* rx;
-  int c, any;
+  double2* X;            // c x c
+  double2* B;            // c x r
+  double2* Y;            // c x (c - r)
+  const double* rx;      // 1 / |x|, by column
+  const int* col;        // the r other columns, then the null ones
+  int c, r;
 };
-__global__ __launch_bounds__(1024) void complete_kernel(const NullJob* __restrict__ jobs) {
-  __shared__ double2 coef[kJacobiMaxCols];
-  __shared__ double part[16];
-  const NullJob J = jobs[blockIdx.x];
-  if (!J.any) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ void null_load_kernel(const NullJob* __restrict__ jobs) {
+  const NullJob J = jobs[blockIdx.y];
   const int64_t c = J.c;
-  int unit = 0;
-  for (int k = 0; k < c; ++k) {
-    if (J.rx[k] != 0.0) continue;
-    double2* const y = J.X + k * c;
-    for (; unit < c; ++unit) {
-      for (int r = tid; r < c; r += 1024) y[r] = make_double2(r == unit ? 1.0 : 0.0, 0.0);
-      __threadfence_block();
-      __syncthreads();
-      for (int pass = 0; pass < 2; ++pass) {
-        for (int j = wave; j < c; j += 16) {
-          const double f = J.rx[j];
-          double gr = 0, gi = 0;
-          if (f != 0.0)
-            for (int r = lane; r < c; r += 64) {
-              const double2 a = J.X[j * c + r], b = y[r];
-              gr += a.x * b.x + a.y * b.y;
-              gi += a.x * b.y - a.y * b.x;
-            }
-          gr = wave_sum(gr);
-          gi = wave_sum(gi);
-          if (lane == 0) coef[j] = make_double2(gr * f * f, gi * f * f);
-        }
-        __syncthreads();
-        for (int r = tid; r < c; r += 1024) {
-          double2 b = y[r];
-          for (int j = 0; j < c; ++j) {
-            const double2 g = coef[j];
-            if (g.x == 0.0 && g.y == 0.0) continue;
-            const double2 p = cmul(J.X[j * c + r], g);
-            b.x -= p.x;
-            b.y -= p.y;
-          }
-          y[r] = b;
-        }
-        __threadfence_block();
-        __syncthreads();
-      }
-      double w = 0.0;
-      for (int r = tid; r < c; r += 1024) w += y[r].x * y[r].x + y[r].y * y[r].y;
-      w = wave_sum(w);
-      if (lane == 0) part[wave] = w;
-      __syncthreads();
-      w = 0.0;
-      for (int q = 0; q < 16; ++q) w += part[q];
-      __syncthreads();
-      if (w > 0.25 / c) {
-        const double f = 1.0 / sqrt(w);
-        for (int r = tid; r < c; r += 1024) y[r] = make_double2(y[r].x * f, y[r].y * f);
-        if (tid == 0) J.rx[k] = 1.0;
-        ++unit;
-        __threadfence_block();
-        __syncthreads();
-        break;
-      }
+  for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < c * c; e += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t i = e % c, k = e / c;
+    if (k < J.r) {
+      const double f = J.rx[J.col[k]];
+      const double2 x = J.X[i + J.col[k] * c];
+      J.B[e] = make_double2(x.x * f, x.y * f);
+    } else {
+      J.Y[i + (k - J.r) * c] = make_double2(i == k ? 1.0 : 0.0, 0.0);
     }
   }
+}
+__global__ void null_store_kernel(const NullJob* __restrict__ jobs) {
+  const NullJob J = jobs[blockIdx.y];
+  const int64_t c = J.c;
+  for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < c * (c - J.r);
+       e += int64_t(gridDim.x) * blockDim.x)
+    J.X[e % c + J.col[J.r + e / c] * c] = J.Y[e];
 }
 
 // singular vectors in falling order: the right ones P W (into Vh or, for
@@ -1131,6 +1095,11 @@ bool jacobi_svd_small(int64_t m, int64_t n) {
 
 bool jacobi_svd_fits(int64_t m, int64_t n) {
   return jacobi_svd_small(m, n) || (std::min(m, n) <= kJacobiMaxCols && std::max(m, n) <= kQrMaxRows);
+}
+
+// columns of a QR panel that fit in LDS, from their rows
+static int panel_width(int64_t rows) {
+  return rows * kB * static_cast<int64_t>(sizeof(double2)) <= kPanelLds ? kB : kB / 2;
 }
 
 std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
@@ -1201,7 +1170,7 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
     Sz z;
     z.L = std::max(it.m, it.n);
     z.c = std::min(it.m, it.n);
-    z.w = z.L * kB * static_cast<int64_t>(sizeof(double2)) <= kPanelLds ? kB : kB / 2;
+    z.w = panel_width(z.L);
     z.npan = (z.c + z.w - 1) / z.w;
     z.nb = static_cast<int>((z.c + kB - 1) / kB);
     z.nb += z.nb & 1;
@@ -1254,6 +1223,7 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
       j.cp = static_cast<int>(z.cp);
       j.w = z.w;
       j.npan = static_cast<int>(z.npan);
+      j.ny = j.c;
       j.scale = scale_of(it.weight);
       qr.push_back(j);
       BlockJob b{};
@@ -1333,7 +1303,7 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
   std::vector<int> hsrc(static_cast<size_t>(ctot));
   std::vector<double> hfac(static_cast<size_t>(2 * ctot));
   std::vector<OutJob> outs(big.size());
-  std::vector<NullJob> nulls(big.size());
+  std::vector<std::vector<int>> null_cols(big.size());
   std::vector<double> hrx(static_cast<size_t>(ctot), 0.0);
   bool vectors = false;
   int64_t cc = 0;
@@ -1344,14 +1314,13 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
     std::iota(ord.begin(), ord.end(), 0);
     const double* nn = hn.data() + 2 * cc;
     ok[big[q]] = jobs[q].done;
-    nulls[q] = NullJob{qr[q].X, dbl.get() + cc, qr[q].c, 0};   // the column lengths' array is free by now
     if (jobs[q].done) {
       std::vector<double> sg(static_cast<size_t>(z.c));
       for (int64_t j = 0; j < z.c; ++j) {
         const bool null = !(nn[2 * j] * nn[2 * j] > kNull2);
         sg[j] = null ? 0.0 : nn[2 * j] / nn[2 * j + 1];
         hrx[cc + j] = null ? 0.0 : 1.0 / nn[2 * j];
-        if (null && it.U) nulls[q].any = 1;
+        if (null && it.U) null_cols[q].push_back(static_cast<int>(j));
       }
       std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return sg[a] > sg[b]; });
       it.S->resize(static_cast<size_t>(z.c));
@@ -1374,11 +1343,66 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
     HIP_CHECK(hipMemcpyAsync(dbl.get() + 3 * ctot, hfac.data(), hfac.size() * sizeof(double), hipMemcpyHostToDevice, s));
     DevBuf<OutJob> dout(outs.size());
     dout.upload(outs.data(), outs.size(), s);
-    DevBuf<NullJob> dz(nulls.size());
-    if (std::any_of(nulls.begin(), nulls.end(), [](const NullJob& n) { return n.any; })) {
+    std::vector<DevBuf<cplx>> completion;
+    DevBuf<NullJob> dz;
+    DevBuf<QrJob> dzq;
+    DevBuf<int> dcol;
+    std::vector<NullJob> nulls;
+    std::vector<QrJob> nqr;
+    std::vector<int> ncol;
+    cc = 0;
+    for (int q = 0; q < nj; ++q) {
+      const int c = qr[q].c, z = static_cast<int>(null_cols[q].size());
+      if (z) {
+        QrJob j{};
+        j.L = c;
+        j.c = c - z;
+        j.w = panel_width(c);
+        j.npan = (j.c + j.w - 1) / j.w;
+        j.ny = z;
+        completion.emplace_back(static_cast<size_t>(c) * c + static_cast<size_t>(j.npan) * kB * kB + j.c);
+        double2* at = reinterpret_cast<double2*>(completion.back().get());
+        j.B = at;
+        j.Y = at + static_cast<int64_t>(c) * j.c;
+        j.T = at + static_cast<int64_t>(c) * c;
+        j.diag = j.T + static_cast<int64_t>(j.npan) * (kB * kB);
+        nqr.push_back(j);
+        // (the column lengths' array is free by now and takes 1 / |x|)
+        nulls.push_back(NullJob{qr[q].X, j.B, j.Y, dbl.get() + cc, nullptr, c, j.c});
+        for (int k = 0, next = 0; k < c; ++k) {
+          if (next < z && null_cols[q][next] == k) ++next;
+          else ncol.push_back(k);
+        }
+        ncol.insert(ncol.end(), null_cols[q].begin(), null_cols[q].end());
+      }
+      cc += c;
+    }
+    if (!nulls.empty()) {
+      const int nn = static_cast<int>(nulls.size());
       HIP_CHECK(hipMemcpyAsync(dbl.get(), hrx.data(), hrx.size() * sizeof(double), hipMemcpyHostToDevice, s));
+      dcol.alloc(ncol.size());
+      dcol.upload(ncol.data(), ncol.size(), s);
+      int pans = 0, off = 0;
+      int64_t nlds = 0;
+      for (int q = 0; q < nn; ++q) {
+        nulls[q].col = dcol.get() + off;
+        off += nulls[q].c;
+        pans = std::max(pans, nqr[q].npan);
+        nlds = std::max(nlds, static_cast<int64_t>(nqr[q].L) * nqr[q].w * static_cast<int64_t>(sizeof(double2)));
+      }
+      dz.alloc(nulls.size());
       dz.upload(nulls.data(), nulls.size(), s);
-      hipLaunchKernelGGL(complete_kernel, dim3(nj), dim3(1024), 0, s, dz.get());
+      dzq.alloc(nqr.size());
+      dzq.upload(nqr.data(), nqr.size(), s);
+      hipLaunchKernelGGL(null_load_kernel, dim3(256, nn), dim3(256), 0, s, dz.get());
+      for (int p = 0; p < pans; ++p) {
+        hipLaunchKernelGGL(panel_kernel, dim3(nn), dim3(kPanelThreads), static_cast<size_t>(nlds), s, dzq.get(), p);
+        hipLaunchKernelGGL(reflect_kernel, dim3(cchunks, nn), dim3(256), 0, s, dzq.get(), p, 0);
+      }
+      for (int p = pans - 1; p >= 0; --p)
+        hipLaunchKernelGGL(reflect_kernel, dim3(cchunks, nn), dim3(256), 0, s, dzq.get(), p, 1);
+      hipLaunchKernelGGL(null_store_kernel, dim3(256, nn), dim3(256), 0, s, dz.get());
+      HIP_CHECK(hipGetLastError());
     }
     hipLaunchKernelGGL(vectors_kernel, dim3(256, nj), dim3(256), 0, s, dq.get(), dout.get());
     for (int p = npan - 1; p >= 0; --p)
