@@ -11,9 +11,9 @@
 // the columns end orthogonal relative to their own lengths, however small.
 // The QR step is there for the spectra of bond wavefunctions: on R^H the
 // rotations need 6 to 9 sweeps, on B itself 15 to 33 (decaying or truncated
-// spectra).  A rotation's rounding drifts the columns' lengths by some 1e-16
-// each, so the singular values are |x_j| / |v_j| and both vectors are
-// normalised at the end.
+// spectra; blocks with repeated columns take a second QR, see kStallSweeps).
+// A rotation's rounding drifts the columns' lengths by some 1e-16 each, so the
+// singular values are |x_j| / |v_j| and both vectors are normalised at the end.
 //
 // Two forms:
 //  - a block whose working set fits the 160 KB of LDS is decomposed by one
@@ -142,6 +142,16 @@ constexpr int64_t kSmallLds = 152 * 1024;
 constexpr int kSmallCols = 72;        // 2 c^2 entries of 16 bytes fit up to c = 69
 constexpr int kSmallRows = 1024;
 constexpr int kMaxSweeps = 40;
+// Blocks (of the block form) whose rotations still meet scaled inner products
+// above kStalled after this many sweeps start again from another QR.  They have
+// columns that repeat others: the QR leaves some copies among the long columns
+// of R^H, where the rotations shrink them by a digit a sweep (128 columns, 64
+// different ones: 36 sweeps; 640 columns, 160 different ones: more than 40).
+// The new QR takes the columns that the first one found dependent last, and
+// entries changed in their last bit: equal columns would leave equal rounding
+// errors, dependent again.  Then 8 to 10 sweeps do.  Other blocks end within 9.
+constexpr int kStallSweeps = 12;
+constexpr double kStalled = 1e-3;
 
 struct SmallJob {
   const double2* A;      // m x n, column-major
@@ -745,6 +755,7 @@ struct QrJob {
   int* perm;             // sorted position -> column
   int m, n, L, c, cp, w, npan, ny;
   double scale;
+  int last_bit;          // whether entries are changed in their last bit
 };
 
 __global__ __launch_bounds__(64) void column_lengths_kernel(const QrJob* __restrict__ jobs) {
@@ -772,6 +783,14 @@ __global__ __launch_bounds__(1024) void sort_columns_kernel(const QrJob* __restr
   }
 }
 
+// x (1 + d), |d| <= eps, pseudorandom by entry
+__device__ __forceinline__ double last_bit(double x, uint64_t e) {
+  e = (e ^ (e >> 30)) * 0xbf58476d1ce4e5b9ull;       // splitmix64's finisher
+  e = (e ^ (e >> 27)) * 0x94d049bb133111ebull;
+  e ^= e >> 31;
+  return x + x * (static_cast<double>(static_cast<int64_t>(e)) * 0x1p-115);
+}
+
 __global__ void load_kernel(const QrJob* __restrict__ jobs) {
   const QrJob J = jobs[blockIdx.y];
   const bool tr = J.m < J.n;
@@ -781,6 +800,7 @@ __global__ void load_kernel(const QrJob* __restrict__ jobs) {
     double2 v = J.A[tr ? k + i * J.m : i + k * J.m];
     v.x *= J.scale;
     v.y *= tr ? -J.scale : J.scale;
+    if (J.last_bit) v = make_double2(last_bit(v.x, 2 * e + 1), last_bit(v.y, 2 * e + 2));
     J.B[e] = v;
   }
 }
@@ -1256,14 +1276,17 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kPanelLds));
   hipLaunchKernelGGL(column_lengths_kernel, dim3(static_cast<unsigned>(cmax), nj), dim3(64), 0, s, dq.get());
   hipLaunchKernelGGL(sort_columns_kernel, dim3(nj), dim3(1024), 0, s, dq.get());
-  hipLaunchKernelGGL(load_kernel, dim3(256, nj), dim3(256), 0, s, dq.get());
   const unsigned cchunks = static_cast<unsigned>((cmax + kB - 1) / kB);
-  for (int p = 0; p < npan; ++p) {
-    hipLaunchKernelGGL(panel_kernel, dim3(nj), dim3(kPanelThreads), static_cast<size_t>(lds), s, dq.get(), p);
-    hipLaunchKernelGGL(reflect_kernel, dim3(cchunks, nj), dim3(256), 0, s, dq.get(), p, 0);
-  }
-  hipLaunchKernelGGL(start_kernel, dim3(256, nj), dim3(256), 0, s, dq.get());
-  HIP_CHECK(hipGetLastError());
+  auto factorise = [&](const QrJob* d, int count) {
+    hipLaunchKernelGGL(load_kernel, dim3(256, count), dim3(256), 0, s, d);
+    for (int p = 0; p < npan; ++p) {
+      hipLaunchKernelGGL(panel_kernel, dim3(count), dim3(kPanelThreads), static_cast<size_t>(lds), s, d, p);
+      hipLaunchKernelGGL(reflect_kernel, dim3(cchunks, count), dim3(256), 0, s, d, p, 0);
+    }
+    hipLaunchKernelGGL(start_kernel, dim3(256, count), dim3(256), 0, s, d);
+    HIP_CHECK(hipGetLastError());
+  };
+  factorise(dq.get(), nj);
   std::vector<unsigned long long> hoff(jobs.size());
   for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
     launch_zero(off.get(), static_cast<int64_t>(jobs.size() * sizeof(unsigned long long)), s);
@@ -1282,6 +1305,7 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
     HIP_CHECK(hipMemcpyAsync(hoff.data(), off.get(), hoff.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     bool all = true;
+    std::vector<QrJob> again;
     for (size_t q = 0; q < jobs.size(); ++q) {
       if (jobs[q].done) continue;
       double w;
@@ -1291,9 +1315,35 @@ std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
       // level nothing was left to rotate
       if (w <= 4.0 * std::numeric_limits<double>::epsilon() * std::sqrt(double(jobs[q].c))) jobs[q].done = 1;
       else all = false;
+      if (sweep + 1 == kStallSweeps && w > kStalled) again.push_back(qr[q]);
     }
     if (all) break;
     dj.upload(jobs.data(), jobs.size(), s);
+    if (again.empty()) continue;
+    for (QrJob& j : again) {
+      const size_t c = static_cast<size_t>(j.c);
+      std::vector<cplx> diag(c);
+      std::vector<int> old(c), order;
+      HIP_CHECK(hipMemcpyAsync(diag.data(), j.diag, c * sizeof(cplx), hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipMemcpyAsync(old.data(), j.perm, c * sizeof(int), hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipStreamSynchronize(s));
+      double longest = 0.0;
+      for (const cplx& d : diag) longest = std::max(longest, std::hypot(d.re, d.im));
+      auto dependent = [&](size_t k) {
+        return std::hypot(diag[k].re, diag[k].im) <= double(c) * std::numeric_limits<double>::epsilon() * longest;
+      };
+      for (size_t k = 0; k < c; ++k)
+        if (!dependent(k)) order.push_back(old[k]);
+      for (size_t k = 0; k < c; ++k)
+        if (dependent(k)) order.push_back(old[k]);
+      HIP_CHECK(hipMemcpyAsync(j.perm, order.data(), c * sizeof(int), hipMemcpyHostToDevice, s));
+      HIP_CHECK(hipStreamSynchronize(s));
+      j.last_bit = 1;
+    }
+    DevBuf<QrJob> da(again.size());
+    da.upload(again.data(), again.size(), s);
+    factorise(da.get(), static_cast<int>(again.size()));
+    HIP_CHECK(hipStreamSynchronize(s));
   }
   hipLaunchKernelGGL(norms_kernel, dim3(static_cast<unsigned>(cmax), nj), dim3(64), 0, s, dq.get(), dn.get());
   HIP_CHECK(hipGetLastError());

@@ -74,8 +74,11 @@ def test_jacobi_rank_deficient(ctx, n, rank):
 # and the largest columns and rows the kernels take.  The rounding grows like
 # the square root of the longer side: sqrt(1200 / 260) = 2.15 times the bounds
 # above, in the Frobenius norm.
-def _check_large(ctx, A):
+def _check_large(ctx, A, monkeypatch, capfd):
+    monkeypatch.setenv("CAM_SVD_TRACE", "1")
+    capfd.readouterr()
     U, s, Vd = _svd(ctx, A)
+    assert "1 of 1 blocks by Jacobi" in capfd.readouterr().err
     ref = np.linalg.svd(A, compute_uv=False)
     k = len(ref)
     assert len(s) == k
@@ -88,15 +91,28 @@ def _check_large(ctx, A):
 
 @pytest.mark.parametrize("m,n", [(600, 70), (601, 70), (70, 601), (1200, 64), (90, 1200), (1200, 9), (640, 600),
                                  (700, 650), (1000, 1024), (1024, 1024)])
-def test_jacobi_large(ctx, m, n):
+def test_jacobi_large(ctx, m, n, monkeypatch, capfd):
     print(f"case jacobi_large m={m} n={n}", flush=True)
     rng = np.random.default_rng(1000 * m + n)
-    _check_large(ctx, _rand(rng, m, n))
+    _check_large(ctx, _rand(rng, m, n), monkeypatch, capfd)
 
 
 @pytest.mark.parametrize("m,n", [(640, 600), (70, 601), (1024, 1000)])
-def test_jacobi_large_rank_deficient(ctx, m, n):
+def test_jacobi_large_rank_deficient(ctx, m, n, monkeypatch, capfd):
     print(f"case jacobi_large_rank_deficient m={m} n={n}", flush=True)
     rng = np.random.default_rng(m + n)
-    _check_large(ctx, _rand(rng, m, 7) @ _rand(rng, 7, n))
-    _check_large(ctx, np.tile(_rand(rng, m, 1), (1, n)) * np.where(np.arange(n) % 2, -1.0, 1.0))
+    _check_large(ctx, _rand(rng, m, 7) @ _rand(rng, 7, n), monkeypatch, capfd)
+    _check_large(ctx, np.tile(_rand(rng, m, 1), (1, n)) * np.where(np.arange(n) % 2, -1.0, 1.0), monkeypatch, capfd)
+
+
+@pytest.mark.parametrize("m,n,different", [(100, 96, 48), (96, 130, 24), (130, 300, 70), (768, 768, 384),
+                                           (1024, 700, 630), (640, 1024, 160), (512, 512, 40)])
+def test_jacobi_repeated_columns(ctx, m, n, different, monkeypatch, capfd):
+    """Columns of the shorter side that repeat others once or more: the
+    rotations get on with such a block only after a second QR."""
+    print(f"case jacobi_repeated_columns m={m} n={n} different={different}", flush=True)
+    rng = np.random.default_rng(m + n)
+    c = min(m, n)
+    A = _rand(rng, max(m, n), different)[:, np.arange(c) % different]
+    A = A * np.where(np.arange(c) // different % 2, -1.0, 1.0)
+    _check_large(ctx, A if m >= n else A.T, monkeypatch, capfd)
