@@ -13,6 +13,11 @@ struct Error : std::runtime_error {
   explicit Error(const std::string& s) : std::runtime_error(s) {}
 };
 
+// device memory exhausted
+struct OutOfMemory : Error {
+  explicit OutOfMemory(const std::string& s) : Error(s) {}
+};
+
 void set_last_error(const std::string& s);
 const char* last_error();
 
@@ -45,7 +50,15 @@ class DevBuf {
   }
   void alloc(size_t n) {
     reset();
-    if (n) HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T)));
+    if (n) {
+      const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T));
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        p_ = nullptr;
+        throw OutOfMemory("HIP error out of memory (hipMalloc of " + std::to_string(n * sizeof(T)) + " bytes)");
+      }
+      HIP_CHECK(e);
+    }
     n_ = n;
   }
   // grow-only (contents not preserved)

@@ -1122,6 +1122,35 @@ static int panel_width(int64_t rows) {
   return rows * kB * static_cast<int64_t>(sizeof(double2)) <= kPanelLds ? kB : kB / 2;
 }
 
+// U and Vh, and the work that jacobi_svd allocates for a block (with the
+// completion of null columns)
+int64_t jacobi_svd_bytes(int64_t m, int64_t n, bool vectors) {
+  const int64_t L = std::max(m, n), c = std::min(m, n), uv = vectors ? (m + n) * c : 0;
+  constexpr int64_t es = sizeof(double2);
+  if (jacobi_svd_small(m, n)) return es * (uv + L * c + c);
+  const int64_t nb = (c + kB - 1) / kB + 1, chunks = (c + kRows - 1) / kRows, pan = c / panel_width(L) + 1;
+  return es * (uv + 2 * L * c + pan * kB * kB + 6 * c + 2 * c * nb * kB + nb / 2 * (chunks + 1) * kP * kP +
+               (vectors ? c * c + pan * kB * kB : 0));
+}
+
+std::vector<size_t> jacobi_svd_batches(const std::vector<JacobiSize>& blocks, bool vectors, int64_t bytes,
+                                       size_t items) {
+  std::vector<size_t> ends;
+  int64_t sum = 0;
+  size_t first = 0;
+  for (size_t i = 0; i < blocks.size(); ++i) {
+    const int64_t b = jacobi_svd_bytes(blocks[i].m, blocks[i].n, vectors);
+    if (i > first && (sum + b > bytes || i - first >= items)) {
+      ends.push_back(i);
+      first = i;
+      sum = 0;
+    }
+    sum += b;
+  }
+  if (first < blocks.size()) ends.push_back(blocks.size());
+  return ends;
+}
+
 std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items) {
   hipStream_t s = ctx.stream;
   std::vector<char> ok(items.size(), 0);

@@ -73,6 +73,15 @@ struct JacobiItem {
 };
 constexpr int64_t kJacobiMaxCols = 1024;
 bool jacobi_svd_fits(int64_t m, int64_t n);
+// Blocks that are decomposed together: ends of consecutive ranges of at most
+// `items` blocks whose vectors and work take at most `bytes` (a block by
+// itself may take more).
+struct JacobiSize { int64_t m, n; };
+constexpr int64_t kJacobiBatchBytes = int64_t(4) << 30;   // some 40 of the largest blocks: 1300 workgroups
+constexpr size_t kJacobiBatchItems = 32768;               // blocks stand in the grid's second dimension
+int64_t jacobi_svd_bytes(int64_t m, int64_t n, bool vectors);
+std::vector<size_t> jacobi_svd_batches(const std::vector<JacobiSize>& blocks, bool vectors,
+                                       int64_t bytes = kJacobiBatchBytes, size_t items = kJacobiBatchItems);
 std::vector<char> jacobi_svd(Ctx& ctx, const std::vector<JacobiItem>& items);
 
 // MPX_matrix::SVD with the reference truncation rule.

@@ -123,18 +123,22 @@ struct WeightJob {
   const double2* p;
   int64_t n;
 };
-__global__ __launch_bounds__(256) void weight_kernel(const WeightJob* __restrict__ jobs, double* __restrict__ out) {
+__global__ __launch_bounds__(256) void weight_kernel(const WeightJob* __restrict__ jobs, int njobs,
+                                                     double* __restrict__ out) {
   __shared__ double part[4];
-  const WeightJob J = jobs[blockIdx.y];
-  double w = 0.0;
-  for (int64_t e = blockIdx.x * int64_t(256) + threadIdx.x; e < J.n; e += int64_t(gridDim.x) * 256) {
-    const double2 v = J.p[e];
-    w += v.x * v.x + v.y * v.y;
+  for (int j = blockIdx.y; j < njobs; j += gridDim.y) {
+    const WeightJob J = jobs[j];
+    double w = 0.0;
+    for (int64_t e = blockIdx.x * int64_t(256) + threadIdx.x; e < J.n; e += int64_t(gridDim.x) * 256) {
+      const double2 v = J.p[e];
+      w += v.x * v.x + v.y * v.y;
+    }
+    for (int o = 32; o > 0; o >>= 1) w += __shfl_down(w, o, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) out[j * int64_t(gridDim.x) + blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+    __syncthreads();
   }
-  for (int o = 32; o > 0; o >>= 1) w += __shfl_down(w, o, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
-  __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.y * int64_t(gridDim.x) + blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
 }
 
 template <typename J, typename K>
@@ -168,7 +172,8 @@ struct Group {
   int64_t first_col = 0;                         // GetAllBlockColumns order key
   double weight = 0.0;
   int64_t k = 0;                                 // number of singular values
-  cplx* A = nullptr;                             // dense compact matrix (in the call's buffer)
+  cplx* A = nullptr;                             // dense compact matrix (own, or in the call's buffer)
+  DevBuf<cplx> Aown;                             // of a block of kOwnElems elements or more
   DevBuf<cplx> U, Vh;                            // the block's own vectors, if not in a shared buffer
   cplx *Up = nullptr, *Vp = nullptr;             // U (mg x k), V^dagger (k x ng)
   std::vector<double> S;
@@ -320,6 +325,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     HIP_CHECK(hipMemcpyAsync(&info, lb.dinfo.get(), sizeof(int), hipMemcpyDeviceToHost, ls));
     HIP_CHECK(hipStreamSynchronize(ls));
     CAM_REQUIRE(info == 0, "blockwise SVD did not converge");
+    g.Aown.reset();
   };
   auto timed_full_svd = [&](Ctx& lane, LaneBufs& lb, Group& g) {
     const auto t1 = std::chrono::steady_clock::now();
@@ -339,13 +345,22 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     bool full;
   };
   std::vector<Pending> pending;
-  // every group's compact dense matrix, gathered in one launch into one buffer
+  // every group's compact dense matrix, gathered in one launch; the large ones
+  // in buffers of their own, which are freed when the group is decomposed, the
+  // others in one
+  constexpr int64_t kOwnElems = int64_t(1) << 16;
   int64_t atot = 0, amax = 0;
   for (Group* g : glist) {
     if (g->mg == 0 || g->ng == 0) continue;
     CAM_REQUIRE(g->mg < (int64_t(1) << 31) && g->ng < (int64_t(1) << 31), "SVD block too large");
-    atot += g->mg * g->ng;
-    amax = std::max(amax, g->mg * g->ng);
+    const int64_t n = g->mg * g->ng;
+    amax = std::max(amax, n);
+    if (n < kOwnElems) {
+      atot += n;
+      continue;
+    }
+    g->Aown.alloc(static_cast<size_t>(n));
+    launch_zero(g->Aown.get(), n * static_cast<int64_t>(sizeof(cplx)), s);
   }
   DevBuf<cplx> abuf(static_cast<size_t>(std::max<int64_t>(atot, 1)));
   launch_zero(abuf.get(), atot * static_cast<int64_t>(sizeof(cplx)), s);
@@ -359,8 +374,11 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     for (Group* gp : glist) {
       Group& g = *gp;
       if (g.mg == 0 || g.ng == 0) continue;
-      g.A = abuf.get() + off;
-      off += g.mg * g.ng;
+      g.A = g.Aown.get();
+      if (!g.A) {
+        g.A = abuf.get() + off;
+        off += g.mg * g.ng;
+      }
       wjobs.push_back(WeightJob{reinterpret_cast<const double2*>(g.A), g.mg * g.ng});
       wgroups.push_back(gp);
       for (int b : g.blocks) {
@@ -412,7 +430,9 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
       DevBuf<WeightJob> dw(wjobs.size());
       dw.upload(wjobs.data(), wjobs.size(), s);
       DevBuf<double> dp(wjobs.size() * static_cast<size_t>(nb));
-      hipLaunchKernelGGL(weight_kernel, dim3(nb, wjobs.size()), dim3(256), 0, s, dw.get(), dp.get());
+      const unsigned gy = static_cast<unsigned>(std::min<size_t>(wjobs.size(), 4096));
+      hipLaunchKernelGGL(weight_kernel, dim3(nb, gy), dim3(256), 0, s, dw.get(), static_cast<int>(wjobs.size()),
+                         dp.get());
       HIP_CHECK(hipGetLastError());
       std::vector<double> hp(wjobs.size() * static_cast<size_t>(nb));
       HIP_CHECK(hipMemcpyAsync(hp.data(), dp.get(), hp.size() * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -448,39 +468,67 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     pending.push_back(Pending{&g, 0, 0, 0, 0.0, false, true});
   }
 
-  // ---- small and middle full decompositions: Jacobi, all in one go ----------
-  DevBuf<cplx> uvbuf;
+  // ---- small and middle full decompositions: Jacobi, as many at a time as
+  // their memory allows ---------------------------------------------------------
+  std::vector<DevBuf<cplx>> uvbufs;
   {
-    std::vector<JacobiItem> items;
-    std::vector<size_t> which;
-    int64_t uv = 0;
+    std::vector<Group*> which;
+    std::vector<JacobiSize> sizes;
+    std::vector<char> done(pending.size(), 0);
+    std::vector<size_t> pos;
     for (size_t q = 0; q < pending.size(); ++q) {
       Group& g = *pending[q].g;
       if (!pending[q].full || !jacobi_svd_fits(g.mg, g.ng) || !std::isfinite(g.weight)) continue;
-      which.push_back(q);
-      uv += (g.mg + g.ng) * std::min(g.mg, g.ng);
+      which.push_back(&g);
+      sizes.push_back(JacobiSize{g.mg, g.ng});
+      pos.push_back(q);
     }
     if (!which.empty()) {
       const auto t1 = std::chrono::steady_clock::now();
-      if (!values_only) uvbuf.alloc(static_cast<size_t>(uv));
-      cplx* at = uvbuf.get();
-      for (size_t q : which) {
-        Group& g = *pending[q].g;
-        g.k = std::min(g.mg, g.ng);
-        if (!values_only) {
-          g.Up = at;
-          g.Vp = at + g.mg * g.k;
-          at += (g.mg + g.ng) * g.k;
+      auto decompose = [&](size_t a, size_t b) {
+        DevBuf<cplx> uvbuf;
+        int64_t uv = 0;
+        for (size_t i = a; i < b; ++i) uv += (sizes[i].m + sizes[i].n) * std::min(sizes[i].m, sizes[i].n);
+        if (!values_only) uvbuf.alloc(static_cast<size_t>(uv));
+        cplx* at = uvbuf.get();
+        std::vector<JacobiItem> items;
+        for (size_t i = a; i < b; ++i) {
+          Group& g = *which[i];
+          g.k = std::min(g.mg, g.ng);
+          if (!values_only) {
+            g.Up = at;
+            g.Vp = at + g.mg * g.k;
+            at += (g.mg + g.ng) * g.k;
+          }
+          items.push_back(JacobiItem{g.A, g.mg, g.ng, g.weight, g.Up, g.Vp, &g.S});
         }
-        items.push_back(JacobiItem{g.A, g.mg, g.ng, g.weight, g.Up, g.Vp, &g.S});
+        const std::vector<char> ok = jacobi_svd(ctx, items);
+        for (size_t i = a; i < b; ++i) {
+          done[pos[i]] = ok[i - a];
+          if (ok[i - a]) which[i]->Aown.reset();
+        }
+        uvbufs.push_back(std::move(uvbuf));
+      };
+      size_t a = 0;
+      for (size_t b : jacobi_svd_batches(sizes, !values_only)) {
+        // without memory for all of them one by one, and a block without memory
+        // for itself is left to the solver below
+        try {
+          decompose(a, b);
+        } catch (const OutOfMemory&) {
+          for (size_t i = a; i < b; ++i) {
+            if (b - a == 1) break;
+            try {
+              decompose(i, i + 1);
+            } catch (const OutOfMemory&) {
+            }
+          }
+        }
+        a = b;
       }
-      const std::vector<char> ok = jacobi_svd(ctx, items);
       std::vector<Pending> rest;
-      for (size_t q = 0, i = 0; q < pending.size(); ++q) {
-        const bool mine = i < which.size() && which[i] == q;
-        if (!(mine && ok[i])) rest.push_back(pending[q]);
-        if (mine) ++i;
-      }
+      for (size_t q = 0; q < pending.size(); ++q)
+        if (!done[q]) rest.push_back(pending[q]);
       if (trace)
         std::fprintf(stderr, "svd_truncate: %zu of %zu blocks by Jacobi, %.6f s\n", pending.size() - rest.size(),
                      pending.size(), std::chrono::duration<double>(std::chrono::steady_clock::now() - t1).count());
@@ -674,6 +722,7 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
                                          glist[gi]->q)] = kept_of[gi];
   }
   abuf.reset();
+  for (Group* g : glist) g->Aown.reset();
   values.clear();
   for (size_t i = 0; i < length; ++i) values.push_back(all[i].v);
   if (values_only) return;

@@ -116,3 +116,24 @@ def test_jacobi_repeated_columns(ctx, m, n, different, monkeypatch, capfd):
     A = _rand(rng, max(m, n), different)[:, np.arange(c) % different]
     A = A * np.where(np.arange(c) // different % 2, -1.0, 1.0)
     _check_large(ctx, A if m >= n else A.T, monkeypatch, capfd)
+
+
+def test_many_blocks(ctx):
+    """90000 blocks of one element: more than a launch's second dimension
+    takes, and several batches."""
+    print("case jacobi many_blocks", flush=True)
+    import chainamps_amd as cam
+    from chainamps_amd.capi import IndexDesc
+    n = 300
+    q = np.stack(np.meshgrid(np.arange(n), np.arange(n), indexing="ij"), -1).reshape(-1, 2) - 150
+    x = np.random.default_rng(9).uniform(0.5, 1.0, n * n) * np.exp(1j * np.arange(n * n))
+    t = cam.Tensor.from_csc(ctx, [0, 0], [IndexDesc(True, False, q), IndexDesc(False, False, q)], 1, n * n, n * n,
+                            np.arange(n * n + 1), np.arange(n * n), x)
+    U, s, Vd, disc = cam.svd_truncate(t, 0, 0.0)
+    order = np.argsort(-np.abs(x), kind="stable")
+    assert np.abs(s - np.abs(x)[order]).max() <= 1e-15
+    rows, cols, p, i, u = U.to_csc()
+    assert np.array_equal(i, order) and np.abs(np.abs(u) - 1.0).max() <= 1e-14
+    rows, cols, p, i, v = Vd.to_csc()
+    k = np.argsort(order)
+    assert np.array_equal(i, k) and np.abs(u[k] * s[k] * v - x).max() <= 1e-14

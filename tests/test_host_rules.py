@@ -1,0 +1,49 @@
+"""CPU: rules the library applies on the host, through a small program linked
+against it (tests/host/host_check.cpp)."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    from chainamps_amd import build
+    from chainamps_amd.capi import library_path
+    lib = library_path()
+    if not lib.exists():
+        pytest.skip("library not built in this checkout (python -m chainamps_amd.build)")
+    exe = tmp_path_factory.mktemp("host") / "host_check"
+    subprocess.run([build.hipcc(), "-std=c++17", "-O1", "-x", "c++", "-D__HIP_PLATFORM_AMD__", f"-I{build.ROCM}/include",
+                    f"-I{ROOT / 'chainamps_amd/csrc'}", str(ROOT / "tests/host/host_check.cpp"), "-o", str(exe),
+                    f"-L{lib.parent}", f"-l:{lib.name}", f"-L{build.ROCM}/lib", "-lamdhip64",
+                    f"-Wl,-rpath,{lib.parent}", f"-Wl,-rpath,{build.ROCM}/lib"], check=True)
+
+    def ask(*lines):
+        r = subprocess.run([str(exe)], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True)
+        return r.stdout.splitlines()
+    return ask
+
+
+def test_svd_batches(check):
+    """Blocks decomposed together stay within the memory and the grid that a
+    call may use, whatever their number; a block that takes more alone."""
+    one = [int(check(f"bytes {v} 1024 1024")[0]) for v in (0, 1)]
+    # vectors: U and Vh; work: R with its reflectors, X and V at least
+    assert one[0] >= 16 * 3 * 1024 ** 2 and one[1] >= one[0] + 16 * 2 * 1024 ** 2
+    for limit, items, blocks in [(3 * one[1], 100, [(1024, 1024)] * 10), (one[1] - 1, 100, [(1024, 1024)] * 3),
+                                 (1 << 40, 4, [(8, 5)] * 11), (one[1], 100, [(9, 4), (1024, 1024), (4, 9), (70, 70)]),
+                                 (1 << 32, 32768, [(2, 2)] * 70000), (1 << 32, 32768, [(1024, 1100)] * 200),
+                                 (1 << 32, 32768, [])]:
+        text = " ".join(f"{m} {n}" for m, n in blocks)
+        ends = [int(x) for x in check(f"batches {limit} {items} 1 {text}")[0].split()]
+        size = {s: int(check(f"bytes 1 {s[0]} {s[1]}")[0]) for s in set(blocks)}
+        assert (ends[-1] if ends else 0) == len(blocks)
+        first = 0
+        for e in ends:
+            assert 0 < e - first <= items
+            assert e - first == 1 or sum(size[s] for s in blocks[first:e]) <= limit
+            first = e
+    assert check(f"batches {1 << 32} 32768 1 " + "384 384 " * 30) == ["30 "]
