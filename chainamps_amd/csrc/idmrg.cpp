@@ -120,9 +120,7 @@ TensorPtr make_prediction(Ctx& ctx, const BSTensor& U, const std::vector<double>
   // . diag(1/prev) from Vd's right bond to U's left bond (same positions)
   CAM_REQUIRE(ALambdaR->idx[2].same_charges(U.idx[1]),
               "prediction: previous left and right bonds carry different charges");
-  std::vector<double> inv(prev.size());
-  for (size_t i = 0; i < prev.size(); ++i) inv[i] = 1.0 / prev[i];
-  scale_along_index(ctx, *ALambdaR, 2, inv);
+  scale_along_index(ctx, *ALambdaR, 2, bond_inverse(ALambdaR->idx[2], prev));
   ALambdaR->idx[2] = U.idx[1];
   ALambdaR->idx[2].inward = false;
   ALambdaR->rebuild_lookup();

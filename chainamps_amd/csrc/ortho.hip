@@ -898,9 +898,7 @@ TensorPtr unit_cell_second(Ctx& ctx, const BSTensor& Vd, const std::vector<doubl
   CAM_REQUIRE(Vd.nidx() == 3, "UnitCell: the row matrix must have three indices");
   TensorPtr A1 = reorder(ctx, Vd, false, {1, 0, 2}, 2);
   scale_along_index(ctx, *A1, 1, values);
-  std::vector<double> inv(previous.size());
-  for (size_t k = 0; k < previous.size(); ++k) inv[k] = 1.0 / previous[k];
-  scale_along_index(ctx, *A1, 2, inv);
+  scale_along_index(ctx, *A1, 2, bond_inverse(A1->idx[2], previous));
   return A1;
 }
 

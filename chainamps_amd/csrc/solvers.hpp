@@ -34,6 +34,9 @@ void gauge_fix(cplx* x, int64_t n, hipStream_t s);
 double entropy(const std::vector<double>& values);
 // contract with a diagonal on index k (values per position of that index)
 void scale_along_index(Ctx& ctx, BSTensor& T, int k, const std::vector<double>& lam);
+// 1 / values of a bond's positions; 0 for null values, those at or below eps
+// times the largest of their charge sector.
+std::vector<double> bond_inverse(const QIndex& bond, const std::vector<double>& values);
 
 // Leading k singular triplets of a dense m x n block (column-major, device)
 // by randomized subspace iteration; true when the Ritz residuals of the

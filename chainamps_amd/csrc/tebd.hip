@@ -40,6 +40,23 @@ __global__ void scale_index_kernel(const ScaleJob* jobs, int njobs) {
 
 }  // namespace
 
+// Without a truncation a rank-deficient bond keeps its null singular values:
+// rounding errors of their block, anywhere from eps times its largest value
+// down to zero.  Their inverses would multiply rounding errors, or be infinite.
+// (A decomposition resolves a block's values to eps times its largest, so the
+// small values of a weak sector are not null.)
+std::vector<double> bond_inverse(const QIndex& bond, const std::vector<double>& values) {
+  CAM_REQUIRE(static_cast<int64_t>(values.size()) == bond.size, "diagonal size mismatch");
+  std::vector<double> inv(values.size());
+  for (const std::vector<int64_t>& sector : bond.sec_pos) {
+    double top = 0.0;
+    for (int64_t p : sector) top = std::max(top, std::fabs(values[p]));
+    for (int64_t p : sector)
+      inv[p] = std::fabs(values[p]) <= std::numeric_limits<double>::epsilon() * top ? 0.0 : 1.0 / values[p];
+  }
+  return inv;
+}
+
 // Multiply a tensor along index k by the diagonal `lam` (one value per
 // position of that index): contract(T, diag MPX, (k,0)) for k the last
 // index keeps the index order (MPX_matrix.cpp:44-54 diagonal constructor).

@@ -398,7 +398,9 @@ int cam_unitcell_destroy(cam_unitcell* u);
  * copies); the basis energies of a cell built on the device are zero.
  * cam_unitcell_from_decomposition: UnitCell(MPSDecomposition, PreviousLambda)
  * (UnitCell.hpp:42-48): [U, diag(values) . Vd . diag(previous)^-1 reordered
- * (phys, in, out)], lambdas [previous, values].
+ * (phys, in, out)], lambdas [previous, values]; null previous values (at or
+ * below 2.2e-16 times the largest of their charge sector) count as zero and
+ * have no inverse: their columns are zero.
  * cam_idmrg_unitcell: the same from an iDMRG object's central decomposition
  * and previous lambda (iDMRG_DRV.cpp:70, getCentralDecomposition /
  * getPreviousLambda).

@@ -1,6 +1,7 @@
 // Host-side rules of the library, driven from tests/test_host_rules.py: one
 // command per line on stdin, one line of answer each.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <iostream>
 #include <map>
@@ -30,8 +31,27 @@ static void bytes(std::istringstream& in) {
   std::printf("%lld\n", static_cast<long long>(jacobi_svd_bytes(m, n, vectors != 0)));
 }
 
+// inverse (CHARGE VALUE)*: inverses of a bond's values
+static void inverse(std::istringstream& in) {
+  QIndex bond;
+  std::vector<double> v;
+  int q;
+  std::string x;
+  while (in >> q >> x) {
+    Charge c;
+    c.q[0] = static_cast<int16_t>(q);
+    bond.charges.push_back(c);
+    v.push_back(std::strtod(x.c_str(), nullptr));
+  }
+  bond.size = static_cast<int64_t>(v.size());
+  bond.build_sectors();
+  for (double y : bond_inverse(bond, v)) std::printf("%.17g ", y);
+  std::printf("\n");
+}
+
 int main() {
-  const std::map<std::string, void (*)(std::istringstream&)> commands = {{"batches", batches}, {"bytes", bytes}};
+  const std::map<std::string, void (*)(std::istringstream&)> commands = {{"batches", batches}, {"bytes", bytes},
+                                                                              {"inverse", inverse}};
   std::string line, name;
   while (std::getline(std::cin, line)) {
     std::istringstream in(line);

@@ -211,3 +211,39 @@ def test_transfer_leading_with_restarts(ctx):
         got, info = cell.transfer_leading(side, ncv=4)
         assert info["converged"] and info["restarts"] > 0, info
         assert abs(got - want) <= 1e-12 * abs(want), (side, got, want, info)
+
+
+def test_unitcell_on_a_rank_deficient_bond(ctx):
+    """A bond cut at nothing (truncation 0) keeps the null values of a
+    rank-deficient matrix; the cell's second matrix is finite all the same,
+    with zero columns there."""
+    print("case ortho cell on a rank-deficient bond", flush=True)
+    import chainamps_amd as cam
+    from chainamps_amd.capi import IndexDesc
+    from chainamps_amd.workloads import tensor_from_dense
+    rng = np.random.default_rng(12)
+    chi, d = 12, 2
+    z = lambda n: np.zeros((n, 1), int)  # noqa: E731
+    c = rng.standard_normal((chi, 1)) + 1j * rng.standard_normal((chi, 1))
+    M = np.tile(c, (1, chi)) * np.where(np.arange(chi) % 2, -1.0, 1.0)
+    prev = cam.svd_truncate(tensor_from_dense(ctx, [0], [IndexDesc(True, False, z(chi)), IndexDesc(False, False, z(chi))],
+                                              1, M / np.linalg.norm(M)), 0, 0.0)[1]
+    assert len(prev) == chi and np.all(prev[1:] <= 1e-15)
+    T = rng.standard_normal((d, chi, d, chi)) + 1j * rng.standard_normal((d, chi, d, chi))
+    idx = [IndexDesc(True, True, z(d)), IndexDesc(True, False, z(chi)), IndexDesc(True, True, z(d)),
+           IndexDesc(False, False, z(chi))]
+    U, s, Vd, _ = cam.svd_truncate(tensor_from_dense(ctx, [0], idx, 2, T / np.linalg.norm(T)), 0, 0.0)
+    A1 = cam.UnitCell.from_decomposition(U, s, Vd, prev).matrix(1)
+
+    def dense(t, shape):
+        rows, cols, p, i, x = t.to_csc()
+        m = np.zeros((cols, rows), complex)
+        m[np.repeat(np.arange(cols), np.diff(p)), i] = x
+        return m.reshape(shape[::-1]).transpose(range(len(shape))[::-1])
+    k = len(s)
+    V = dense(Vd, (k, d, chi))                            # [new, s, a_r]
+    keep = prev > 2.220446049250313e-16 * prev.max()
+    inv = np.where(keep, 1.0 / np.where(keep, prev, 1.0), 0.0)
+    ref = V.transpose(1, 0, 2) * s[:, None] * inv
+    got = dense(A1, (d, k, chi))
+    assert np.isfinite(got).all() and np.abs(got - ref).max() <= 1e-14 * np.abs(ref).max()

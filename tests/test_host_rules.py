@@ -47,3 +47,18 @@ def test_svd_batches(check):
             assert e - first == 1 or sum(size[s] for s in blocks[first:e]) <= limit
             first = e
     assert check(f"batches {1 << 32} 32768 1 " + "384 384 " * 30) == ["30 "]
+
+
+def test_bond_inverse(check):
+    """Null values of a charge sector have no inverse; the small values of a
+    weak sector, negative and not-finite ones do."""
+    def inv(*pairs):
+        return [float(x) for x in check("inverse " + " ".join(f"{q} {v!r}" for q, v in pairs))[0].split()]
+    assert inv((0, 0.5), (0, 0.25)) == [2.0, 4.0]
+    assert inv((0, 1.0), (0, 0.0), (0, 1e-40), (0, 2.2e-16), (0, 2.3e-16)) == [1.0, 0.0, 0.0, 0.0, 1 / 2.3e-16]
+    assert inv((0, 1.0), (1, 1e-18), (0, 1e-18), (1, 1e-30), (1, 1e-35)) == [1.0, 1 / 1e-18, 0.0, 1 / 1e-30, 0.0]
+    assert inv((0, 0.0), (0, 0.0)) == [0.0, 0.0]
+    assert inv((0, -0.5), (0, -1e-20)) == [-2.0, 0.0]
+    assert inv((0, float("inf")), (1, 2.0)) == [0.0, 0.5]
+    x = inv((0, float("nan")), (1, 2.0))
+    assert x[0] != x[0] and x[1] == 0.5
