@@ -119,8 +119,7 @@ def test_jacobi_repeated_columns(ctx, m, n, different, monkeypatch, capfd):
 
 
 def test_many_blocks(ctx):
-    """90000 blocks of one element: more than a launch's second dimension
-    takes, and several batches."""
+    """90000 blocks of one element: three batches."""
     print("case jacobi many_blocks", flush=True)
     import chainamps_amd as cam
     from chainamps_amd.capi import IndexDesc
