@@ -828,16 +828,21 @@ int GemmPlan::add_problem(void* C, int64_t csC, int M, int N, int batch, int64_t
   p.cspace = cspace;
   probs.push_back(p);
   group.push_back(-1);
-  uploaded = rows_built = false;
-  for (int m = 0; m < kTileModes; ++m) built[m] = tiles_uploaded[m] = false;
+  uploaded = false;
+  changed();
   return static_cast<int>(probs.size()) - 1;
+}
+
+void GemmPlan::changed() {
+  rows_built = direct_uploaded = false;
+  direct.clear();
+  for (int m = 0; m < kTileModes; ++m) built[m] = tiles_uploaded[m] = false;
 }
 
 void GemmPlan::set_group(int prob, int64_t g) {
   CAM_REQUIRE(prob >= 0 && prob < static_cast<int>(probs.size()), "set_group: no such problem");
   group[prob] = g;
-  rows_built = false;
-  for (int m = 0; m < kTileModes; ++m) built[m] = tiles_uploaded[m] = false;
+  changed();
 }
 
 void GemmPlan::add_segment(int prob, const void* A, int64_t csA, int64_t bsA, const void* B,
@@ -869,7 +874,8 @@ void GemmPlan::add_segment(int prob, const void* A, int64_t csA, int64_t bsA, co
   segs.push_back(g);
   p.nseg++;
   flops += 8.0 * double(p.M) * double(p.N) * double(K) * double(p.batch);
-  uploaded = rows_built = false;
+  uploaded = false;
+  changed();
 }
 
 void GemmPlan::choose_tiles(int mode) {

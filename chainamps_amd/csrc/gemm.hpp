@@ -189,6 +189,8 @@ struct GemmPlan {
   // Histogram signature: problems bucketed by (log2 M, log2 N, log2 K,
   // batched), weighted by flops (5% steps), plus the precision.
   uint64_t signature(int precision) const;
+  // drops every list of a plan that is being added to
+  void changed();
   // problems, segments and every built tile list to the device
   void upload(hipStream_t s);
   // whether a launch at this precision finds all it needs on the device

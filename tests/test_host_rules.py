@@ -62,3 +62,31 @@ def test_bond_inverse(check):
     assert inv((0, float("inf")), (1, 2.0)) == [0.0, 0.5]
     x = inv((0, float("nan")), (1, 2.0))
     assert x[0] != x[0] and x[1] == 0.5
+
+
+def _problem(m, n, ks, batch=1, beta=0):
+    return f"{m} {n} {batch} {beta} {len(ks)} " + " ".join(map(str, ks))
+
+
+def test_plans_cover_their_outputs(check):
+    """Whichever kernels a grouped plan goes to, every output is computed
+    once, at sizes around the tiles, the row passes and the k shares."""
+    seen = set()
+    for ps in [[(1, 1, [1])], [(17, 33, [3])], [(65, 63, [33])], [(200, 18, [257])], [(129, 130, [100])],
+               [(1025, 13, [29])], [(16, 16, [32, 32, 7])], [(16, 17, [32])], [(40, 5, [8], 37), (40, 5, [8], 37)],
+               [(300, 300, [16]), (300, 300, [700])], [(1000, 700, [200])], [(70, 3, [4, 4]), (70, 130, [9])],
+               [(33, 17, [1]), (5, 129, [33]), (31, 15, [65]), (16, 16, [129])], [(64, 20, [300], 3, 1)],
+               [(7, 9, [])], [(512, 512, [10000])]]:
+        probs = [_problem(p[0], p[1], p[2], *p[3:]) for p in ps]
+        route, lo, hi = check("plan " + " ".join(probs))[0].split()
+        assert (lo, hi) == ("1", "1"), (ps, route, lo, hi)
+        seen.add(route)
+    assert seen == {"direct", "tiles", "rows", "tiles+rows"}
+
+
+def test_plan_extended_after_its_lists(check):
+    """A problem added to a plan whose lists are built is not left out."""
+    a, b = _problem(200, 18, [257]), _problem(100, 40, [300])
+    assert check("plan " + a)[0] == "direct 1 1"
+    assert check(f"plan {a} + {b}")[0].split()[1:] == ["1", "1"]
+    assert check(f"plan {_problem(1000, 700, [200])} + {b}")[0].split()[1:] == ["1", "1"]
