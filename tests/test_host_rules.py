@@ -76,7 +76,7 @@ def test_plans_cover_their_outputs(check):
                [(1025, 13, [29])], [(16, 16, [32, 32, 7])], [(16, 17, [32])], [(40, 5, [8], 37), (40, 5, [8], 37)],
                [(300, 300, [16]), (300, 300, [700])], [(1000, 700, [200])], [(70, 3, [4, 4]), (70, 130, [9])],
                [(33, 17, [1]), (5, 129, [33]), (31, 15, [65]), (16, 16, [129])], [(64, 20, [300], 3, 1)],
-               [(7, 9, [])], [(512, 512, [10000])]]:
+               [(2000, 16, [32]), (1000, 700, [200])], [(7, 9, [])], [(512, 512, [10000])]]:
         probs = [_problem(p[0], p[1], p[2], *p[3:]) for p in ps]
         route, lo, hi = check("plan " + " ".join(probs))[0].split()
         assert (lo, hi) == ("1", "1"), (ps, route, lo, hi)
