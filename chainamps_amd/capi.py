@@ -82,6 +82,7 @@ _SIGS = {
     "cam_heff_get_slices": [_p, C.POINTER(C.c_int), C.POINTER(C.c_int), _dp],
     "cam_heff_set_launch": [_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int],
     "cam_heff_get_launch": [_p, C.c_int, C.POINTER(C.c_int)],
+    "cam_heff_get_route": [_p, C.c_int, C.POINTER(C.c_int)],
     "cam_heff_stage_bytes": [_p, _dp],
     "cam_heff_to_blocked": [_p, _p, _p],
     "cam_heff_from_blocked": [_p, _p, _p],
@@ -402,6 +403,13 @@ class Heff:
         cfg = np.zeros(16, np.int32)
         _check(_LIB.cam_heff_get_launch(self.h, precision, _ptr(cfg, C.c_int)))
         return [tuple(int(v) for v in cfg[4 * i:4 * i + 4]) for i in range(4)]
+
+    def get_route(self, precision=CAM_FP64):
+        """Kernels of the stages L, W, W, R: 1 tiles, 2 row passes, 4 the
+        one-launch kernel of small plans (sums)."""
+        r = np.zeros(4, np.int32)
+        _check(_LIB.cam_heff_get_route(self.h, precision, _ptr(r, C.c_int)))
+        return [int(v) for v in r]
 
     def to_blocked(self, din, dout):
         _check(_LIB.cam_heff_to_blocked(self.h, din, dout))

@@ -416,6 +416,17 @@ int cam_heff_get_launch(const cam_heff* h, int precision, int* cfg) {
   CAM_API_END
 }
 
+int cam_heff_get_route(const cam_heff* h, int precision, int* route) {
+  CAM_API_BEGIN
+  CAM_REQUIRE(h && route, "null argument");
+  CAM_REQUIRE(precision == CAM_FP64 || precision == CAM_FP32, "bad precision");
+  for (int i = 0; i < 4; ++i) {
+    route[i] = 0;
+    for (const auto& st : h->h.plans) route[i] |= st[i].route(precision);
+  }
+  CAM_API_END
+}
+
 int cam_heff_to_blocked(cam_heff* h, const double* in_dev, double* out_dev) {
   CAM_API_BEGIN
   set_device(h->owner);

@@ -1241,6 +1241,15 @@ void GemmPlan::upload(hipStream_t s) {
   for (int m = 0; m < kTileModes; ++m) tiles_uploaded[m] = built[m];
 }
 
+int GemmPlan::route(int precision) const {
+  const LaunchCfg& c = cfg[precision];
+  if (c.direct && !direct.empty()) return 4;
+  int r = rows.empty() ? 0 : 2;
+  for (const auto& t : tiles[c.tile_mode])
+    if (!t.empty()) r |= 1;
+  return r;
+}
+
 bool GemmPlan::on_device(int precision) const {
   const LaunchCfg& c = cfg[precision];
   if (c.direct && !direct.empty()) return uploaded && direct_uploaded;
@@ -1309,7 +1318,10 @@ bool autotune(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bas
   if ((e && *e == '0') || plan.flops < min_flops) return false;
   for (const GemmProb& p : plan.probs)
     CAM_REQUIRE(!p.beta, "autotune: a plan that accumulates into its output cannot be re-run");
-  const uint64_t key = plan.signature(precision);
+  // (a plan with few outputs and a long K can be small and be tuned; what a
+  // plan without the choice found does not decide it)
+  const bool small = !plan.direct.empty();
+  const uint64_t key = plan.signature(precision) ^ (small ? 0x9e3779b97f4a7c15ull : 0);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune_cache.find(key);
@@ -1337,10 +1349,16 @@ bool autotune(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bas
     }
     return best;
   };
-  // (a plan large enough to be tuned is never a small one)
+  LaunchCfg cur = plan.cfg[precision];
+  // a small plan: the one-launch kernel against the best tiles
+  float tdirect = 1e30f;
+  if (small) {
+    cur.direct = true;
+    tdirect = time_it(cur);
+    cur.direct = false;
+  }
   // coordinate descent: product form, then tile policy, then K chunk, then
   // grid size
-  LaunchCfg cur = plan.cfg[precision];
   float tcur = time_it(cur);
   auto try_axis = [&](int LaunchCfg::*field, std::initializer_list<int> vals) {
     for (int v : vals) {
@@ -1355,6 +1373,7 @@ bool autotune(GemmPlan& plan, int precision, hipStream_t s, const GemmBases* bas
   try_axis(&LaunchCfg::tile_mode, {1, 0, 2, 3});
   try_axis(&LaunchCfg::kc, {16, 8});
   try_axis(&LaunchCfg::wg_per_cu, {4, 2, 8});
+  if (tdirect < tcur) cur.direct = true;
   apply_choice(plan, precision, cur, s);
   // leave the output of the chosen configuration (every candidate computes
   // the same values; this keeps the last write consistent with the choice)

@@ -193,6 +193,9 @@ struct GemmPlan {
   void changed();
   // problems, segments and every built tile list to the device
   void upload(hipStream_t s);
+  // what a launch at this precision runs: 1 tiles, 2 row passes, 4 the kernel
+  // of small plans (summed)
+  int route(int precision) const;
   // whether a launch at this precision finds all it needs on the device
   bool on_device(int precision) const;
   void clear();

@@ -196,6 +196,10 @@ int cam_heff_stage_bytes(const cam_heff* h, double* stage_bytes);
  * get returns {algo, tile_mode, wg_per_cu, kchunk} per stage (16 ints). */
 int cam_heff_set_launch(cam_heff* h, int precision, int algo, int tile_mode, int wg_per_cu, int kchunk);
 int cam_heff_get_launch(const cam_heff* h, int precision, int* cfg);
+/* The kernels of each stage (4 ints) at the current configuration: 1 tiles,
+ * 2 row passes, 4 the one-launch kernel of small plans (sums; a plan takes the
+ * last by default, where set_launch selects tiles and row passes). */
+int cam_heff_get_route(const cam_heff* h, int precision, int* route);
 /* Reference order <-> device block layout (K3 gather/scatter). */
 int cam_heff_to_blocked(cam_heff* h, const double* in_dev, double* out_dev);
 int cam_heff_from_blocked(cam_heff* h, const double* in_dev, double* out_dev);

@@ -74,3 +74,36 @@ def test_noalloc(ctx):
     finally:
         for b in (x, y, z):
             b.free()
+
+
+def test_tuned(ctx):
+    """A plan of few outputs and a long K is small and yet large enough to be
+    tuned (2e10 flops): the one-launch kernel is one of the candidates, and
+    both precisions end on a configuration that computes the same."""
+    print("case small_plan tuned", flush=True)
+    import chainamps_amd as cam
+    chi, d, w = 214, 2, 64
+    rng = np.random.default_rng(chi)
+    (L, W, R), ups = _env(rng, chi, d, w)
+    psi = _rand(rng, d, chi, d, chi)                       # [s1, a0, s2, a2]
+    t = np.einsum("xba,iajc->xbijc", L, psi, optimize=True)
+    t = np.einsum("pbiq,xbijc->xqpjc", W, t, optimize=True)
+    t = np.einsum("rqjs,xqpjc->xsprc", W, t, optimize=True)
+    ref = np.einsum("xsprc,ysc->pxry", t, R, optimize=True)
+    flat = lambda T: T.transpose(3, 2, 1, 0).reshape(-1)   # noqa: E731  first index fastest
+    v, out_ref = flat(psi), flat(ref)
+    H = cam.Heff(*(u(ctx) for u in ups))
+    # K of the last stage is 64 x 214: rounding grows with its square root
+    for prec, tol in ((cam.CAM_FP64, 1e-12), (cam.CAM_FP32, 1e-4)):
+        assert H.get_route(prec)[3] == 4                   # small until it is tuned
+        assert rel_err(H.apply(v, prec), out_ref) <= tol, prec
+        print("  launch", H.get_launch(prec), "route", H.get_route(prec), flush=True)
+        assert all(r in (1, 2, 3, 4) for r in H.get_route(prec))
+        assert rel_err(H.apply(v, prec), out_ref) <= tol, prec
+        # the tiles that the tuning left for a plan without the choice
+        algo, mode, wg, kc = H.get_launch(prec)[3]
+        T = cam.Heff(*(u(ctx) for u in ups))
+        T.set_launch(prec, algo, mode, wg, kc)
+        assert T.get_route(prec)[3] == 1
+        assert rel_err(T.apply(v, prec), out_ref) <= tol, prec
+        print("  stage ms tuned", H.profile(prec, 5), "tiles", T.profile(prec, 5), flush=True)
