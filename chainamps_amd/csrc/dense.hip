@@ -20,6 +20,7 @@
 // this route with up to 900 entries: 545 -> 23 ms.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <limits>
 
 #include "solvers.hpp"
@@ -211,6 +212,14 @@ double tridiagonal_lowest(const std::vector<double>& a, const std::vector<double
     lo = std::min(lo, a[i] - r);
     hi = std::min(hi, a[i]);              // the lowest eigenvalue is at most every diagonal entry
     nrm = std::max(nrm, std::fabs(a[i]) + r);
+  }
+  // squares of the entries stay in range
+  const int scale = nrm > 0.0 ? std::ilogb(nrm) : 0;
+  if (std::abs(scale) > 400) {
+    std::vector<double> sa(a), sb(b);
+    for (double& x : sa) x = std::ldexp(x, -scale);
+    for (double& x : sb) x = std::ldexp(x, -scale);
+    return std::ldexp(tridiagonal_lowest(sa, sb, vec), scale);
   }
   const double tiny = std::max(eps * eps * nrm, std::numeric_limits<double>::min());
   auto below = [&](double x) {            // whether an eigenvalue is < x

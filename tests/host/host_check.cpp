@@ -50,6 +50,26 @@ static void inverse(std::istringstream& in) {
   std::printf("\n");
 }
 
+// tridiagonal K A.. B..: lowest eigenvalue, then its vector
+static void tridiagonal(std::istringstream& in) {
+  size_t k;
+  in >> k;
+  auto read = [&](size_t n) {
+    std::vector<double> v;
+    std::string x;
+    while (n--) {
+      in >> x;
+      v.push_back(std::strtod(x.c_str(), nullptr));
+    }
+    return v;
+  };
+  const std::vector<double> a = read(k), b = read(k - 1);
+  std::vector<double> vec;
+  std::printf("%.17g ", tridiagonal_lowest(a, b, vec));
+  for (double x : vec) std::printf("%.17g ", x);
+  std::printf("\n");
+}
+
 // Problems of a plan, "M N BATCH BETA NSEG K.." each: what computes its outputs
 // (kernels in route order) and how often each output is computed at least and
 // at most.  A problem after "+" is added when the lists have been built.
@@ -123,7 +143,8 @@ static void plan(std::istringstream& in) {
 int main() {
   const std::map<std::string, void (*)(std::istringstream&)> commands = {{"batches", batches}, {"bytes", bytes},
                                                                               {"inverse", inverse},
-                                                                              {"plan", plan}};
+                                                                              {"plan", plan},
+                                                                              {"tridiagonal", tridiagonal}};
   std::string line, name;
   while (std::getline(std::cin, line)) {
     std::istringstream in(line);

@@ -3,6 +3,7 @@ against it (tests/host/host_check.cpp)."""
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -90,3 +91,24 @@ def test_plan_extended_after_its_lists(check):
     assert check("plan " + a)[0] == "direct 1 1"
     assert check(f"plan {a} + {b}")[0].split()[1:] == ["1", "1"]
     assert check(f"plan {_problem(1000, 700, [200])} + {b}")[0].split()[1:] == ["1", "1"]
+
+
+def test_tridiagonal_lowest(check):
+    """Lowest eigenpair of a symmetric tridiagonal matrix against numpy:
+    random, decoupled, degenerate and zero matrices, at scales down to and up
+    to those whose squares leave the range of a double."""
+    rng = np.random.default_rng(4)
+    cases = [(rng.standard_normal(k), rng.standard_normal(max(k - 1, 0))) for k in (1, 2, 3, 20, 63)]
+    cases += [(np.array([2.0, 1.0, 3.0]), np.zeros(2)), (np.zeros(4), np.zeros(3)), (np.ones(5), np.zeros(4)),
+              (np.full(30, -1.0), np.full(29, 1e-9)), (np.arange(40.0), np.full(39, 1e-3))]
+    for scale in (1.0, 1e150, 1e-150, 1e250, 1e-250):
+        for a, b in cases:
+            k = len(a)
+            out = check(f"tridiagonal {k} " + " ".join(repr(float(x) * scale) for x in np.concatenate([a, b])))
+            got = np.array([float(x) for x in out[0].split()])
+            e, v = got[0] / scale, got[1:]
+            T = np.diag(a) + np.diag(b, 1) + np.diag(b, -1)
+            nrm = max(np.abs(T).sum(1).max(), 1e-300)
+            assert abs(np.linalg.norm(v) - 1.0) <= 1e-14
+            assert abs(e - np.linalg.eigvalsh(T)[0]) <= 4e-15 * nrm, (scale, k)
+            assert np.linalg.norm(T @ v - e * v) <= 1e-14 * nrm, (scale, k)
