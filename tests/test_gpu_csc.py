@@ -43,3 +43,16 @@ def test_csc(ctx, sizes, charges, numrows):
         assert np.array_equal(p, np.concatenate([[0], np.cumsum(np.bincount(c, minlength=cols))]))
         assert np.array_equal(i, r)
         assert np.array_equal(x.view(np.float64), m[c, r].view(np.float64), equal_nan=True)
+
+
+@pytest.mark.parametrize("sizes,charges", [((2300, 2401), (1, 1)), ((3300, 3400), (2, 2))])
+def test_csc_chunks(ctx, sizes, charges):
+    """More stored entries than are emitted at a time (2^22)."""
+    print(f"case csc chunks {sizes} {charges}", flush=True)
+    T, t = _tensor(ctx, sizes, charges, [True, False], 1, 3)
+    rows, cols, p, i, x = t.to_csc()
+    c, r = np.nonzero(T.T)
+    assert len(x) > 1 << 22 and len(c) == len(x)
+    assert np.array_equal(p, np.concatenate([[0], np.cumsum(np.bincount(c, minlength=cols))]))
+    assert np.array_equal(i, r)
+    assert np.array_equal(x.view(np.float64), T.T[c, r].view(np.float64))

@@ -89,3 +89,26 @@ def test_heff_every_launch(ctx, chi, d, w):
                 for kc in (8, 16):
                     H.set_launch(prec, algo=algo, tile_mode=mode, wg_per_cu=2, kchunk=kc)
                     assert rel_err(H.apply(v, prec), out_ref) <= tol, (prec, algo, mode, kc)
+
+
+# Blocks that go to the tiles (test_host_rules.py holds the rule to that) with
+# several K chunks of 8 and a remainder: conjugated operands through the whole
+# pipelined loop.  (Of the sizes above the last two are small plans.)
+TILE_SIZES = [(700, 650, 100), (1025, 515, 257), (333, 1500, 129), (513, 700, 75), (97, 1025, 49), (1537, 161, 97)]
+
+
+@pytest.mark.parametrize("m,n,k", TILE_SIZES)
+@pytest.mark.parametrize("conjA,conjB", [(False, False), (True, False), (False, True), (True, True)])
+def test_contract_tiles(ctx, m, n, k, conjA, conjB):
+    test_contract_edges(ctx, m, n, k, conjA, conjB)
+
+
+def test_heff_routes(ctx):
+    """The launches of test_heff_every_launch run the tiles (its narrow W
+    stages row passes)."""
+    import chainamps_amd as cam
+    for chi, d, w in [(131, 3, 2), (66, 33, 2), (129, 17, 1)]:
+        H = cam.Heff(*(u(ctx) for u in _env(np.random.default_rng(chi), chi, d, w)[1]))
+        for prec in (cam.CAM_FP64, cam.CAM_FP32):
+            H.set_launch(prec, algo=0, tile_mode=1, wg_per_cu=2, kchunk=8)
+            assert H.get_route(prec) == ([1, 2, 2, 1] if d == 3 else [1, 1, 1, 1])

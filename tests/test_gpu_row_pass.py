@@ -63,3 +63,12 @@ def test_heff(ctx, chi, d, w):
         assert rel_err(H.apply(v, prec), out_ref) <= tol, prec
     H.set_slices(2, 2)                                     # accumulating passes
     assert rel_err(H.apply(v), out_ref) <= 1e-13
+
+
+def test_routes(ctx):
+    """The W stages of the cases above run as row passes, past the largest
+    number of inputs as something else."""
+    import chainamps_amd as cam
+    for chi, d, w in [(3, 1, 1), (7, 2, 5), (21, 5, 6), (12, 3, 30), (9, 16, 5), (5, 16, 12), (5, 16, 13)]:
+        H = cam.Heff(*(u(ctx) for u in _env(np.random.default_rng(chi), chi, d, w)[1]))
+        assert all((r == 2) == (d * w <= 192) for r in H.get_route()[1:3]), (chi, d, w)

@@ -107,3 +107,20 @@ def test_tuned(ctx):
         assert T.get_route(prec)[3] == 1
         assert rel_err(T.apply(v, prec), out_ref) <= tol, prec
         print("  stage ms tuned", H.profile(prec, 5), "tiles", T.profile(prec, 5), flush=True)
+
+
+def test_routes(ctx):
+    """The cases above run the one-launch kernel before set_launch, and tiles
+    or row passes after it."""
+    import chainamps_amd as cam
+    from chainamps_amd import workloads
+    for chi, d, w in [(17, 1, 2), (31, 2, 3), (33, 1, 17), (64, 1, 5), (65, 2, 3), (100, 1, 4), (2, 40, 3), (1, 65, 2),
+                      (200, 1, 2)]:
+        H = cam.Heff(*(u(ctx) for u in _env(np.random.default_rng(chi), chi, d, w)[1]))
+        for prec in (cam.CAM_FP64, cam.CAM_FP32):
+            assert 4 in H.get_route(prec), (chi, d, w)
+            H.set_launch(prec, algo=0, tile_mode=1, wg_per_cu=4, kchunk=16)
+            assert 4 not in H.get_route(prec), (chi, d, w)
+    for chi in (90, 160):
+        H = cam.Heff(*workloads.coupled_chain_heff_inputs(ctx, chi=chi, d=2, seed=chi, Jperp=0.3, hermitian=False))
+        assert 4 in H.get_route(), chi

@@ -112,3 +112,16 @@ def test_tridiagonal_lowest(check):
             assert abs(np.linalg.norm(v) - 1.0) <= 1e-14
             assert abs(e - np.linalg.eigvalsh(T)[0]) <= 4e-15 * nrm, (scale, k)
             assert np.linalg.norm(T @ v - e * v) <= 1e-14 * nrm, (scale, k)
+
+
+def test_routes_of_the_contraction_tests(check):
+    """The sizes at which the GPU tests of a kernel contract reach that
+    kernel."""
+    from test_gpu_gemm_edges import TILE_SIZES
+    route = lambda m, n, k: check("plan " + _problem(m, n, [k]))[0].split()[0]  # noqa: E731
+    assert {route(*s) for s in TILE_SIZES} == {"tiles"}
+    assert {route(*s) for s in [(1, 17, 1), (17, 33, 3), (31, 64, 15), (32, 65, 16), (33, 20, 17), (64, 96, 31),
+                                (65, 63, 33)]} == {"tiles"}
+    assert {route(*s) for s in [(129, 130, 100), (200, 18, 257)]} == {"direct"}
+    assert {route(*s) for s in [(1, 1, 1), (15, 16, 4), (16, 15, 5), (17, 1, 3), (63, 2, 31), (65, 16, 32), (1023, 7, 8),
+                                (1025, 13, 29)]} == {"rows"}
