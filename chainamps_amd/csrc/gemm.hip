@@ -824,7 +824,6 @@ int GemmPlan::add_problem(void* C, int64_t csC, int M, int N, int batch, int64_t
   p.nseg = 0;
   p.batch = batch;
   p.beta = beta;
-  p.tile = 0;
   p.cspace = cspace;
   probs.push_back(p);
   group.push_back(-1);

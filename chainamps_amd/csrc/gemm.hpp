@@ -59,7 +59,6 @@ struct GemmProb {
   int32_t seg0, nseg;
   int32_t batch;
   int32_t beta;       // 1: accumulate into C
-  int32_t tile;       // tile shape id (see kTileShapes)
   int32_t cspace;     // operand space of C
 };
 
