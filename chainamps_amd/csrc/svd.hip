@@ -173,7 +173,7 @@ struct Group {
   double weight = 0.0;
   int64_t k = 0;                                 // number of singular values
   cplx* A = nullptr;                             // dense compact matrix (own, or in the call's buffer)
-  DevBuf<cplx> Aown;                             // of a block of kOwnElems elements or more
+  DevBuf<cplx> Aown;                             // of a large block
   DevBuf<cplx> U, Vh;                            // the block's own vectors, if not in a shared buffer
   cplx *Up = nullptr, *Vp = nullptr;             // U (mg x k), V^dagger (k x ng)
   std::vector<double> S;
@@ -345,17 +345,20 @@ void svd_core(Ctx& ctx, const BSTensor& th, int64_t D, double max_trunc, TensorP
     bool full;
   };
   std::vector<Pending> pending;
-  // every group's compact dense matrix, gathered in one launch; the large ones
-  // in buffers of their own, which are freed when the group is decomposed, the
-  // others in one
-  constexpr int64_t kOwnElems = int64_t(1) << 16;
-  int64_t atot = 0, amax = 0;
+  // every group's compact dense matrix, gathered in one launch into one buffer;
+  // of more than 256 MB the large ones into buffers of their own, which are
+  // freed when the group is decomposed (below that an allocation and a free per
+  // block cost more than the memory is worth: two blocks of 384^2 16.45 ms
+  // against 16.23)
+  constexpr int64_t kOwnElems = int64_t(1) << 16, kOwnTotal = int64_t(1) << 24;
+  int64_t atot = 0, amax = 0, all_elems = 0;
+  for (const Group* g : glist) all_elems += g->mg * g->ng;
   for (Group* g : glist) {
     if (g->mg == 0 || g->ng == 0) continue;
     CAM_REQUIRE(g->mg < (int64_t(1) << 31) && g->ng < (int64_t(1) << 31), "SVD block too large");
     const int64_t n = g->mg * g->ng;
     amax = std::max(amax, n);
-    if (n < kOwnElems) {
+    if (n < kOwnElems || all_elems <= kOwnTotal) {
       atot += n;
       continue;
     }

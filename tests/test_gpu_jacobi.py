@@ -136,3 +136,22 @@ def test_many_blocks(ctx):
     rows, cols, p, i, v = Vd.to_csc()
     k = np.argsort(order)
     assert np.array_equal(i, k) and np.abs(u[k] * s[k] * v - x).max() <= 1e-14
+
+
+def test_large_blocks_together(ctx):
+    """Eighteen blocks of 990 x 1000 (285 MB): each in a buffer of its own."""
+    print("case jacobi large_blocks_together", flush=True)
+    import chainamps_amd as cam
+    from chainamps_amd.capi import IndexDesc
+    m, n, k = 990, 1000, 18
+    A = _rand(np.random.default_rng(21), m, n)
+    scale = np.linspace(1.0, 2.0, k)
+    x = (scale[:, None, None] * A.T).reshape(-1)
+    rows = (np.arange(k)[:, None, None] * m + np.zeros((n, 1), int) + np.arange(m)).reshape(-1)
+    q = lambda s: np.repeat(np.arange(k), s).reshape(-1, 1)  # noqa: E731
+    t = cam.Tensor.from_csc(ctx, [0], [IndexDesc(True, False, q(m)), IndexDesc(False, False, q(n))], 1, m * k, n * k,
+                            np.arange(n * k + 1) * m, rows, x)
+    s = cam.svd_truncate(t, 0, 0.0)[1]
+    ref = np.linalg.svd(A, compute_uv=False)
+    ref = np.sort(np.outer(scale, ref).reshape(-1))[::-1]
+    assert len(s) == m * k and np.abs(s - ref).max() <= 2.2e-13 * ref[0]
