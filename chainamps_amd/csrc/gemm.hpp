@@ -11,8 +11,9 @@
 // interleaved (re,im); a complex multiply runs as three (Gauss) or four real
 // MFMAs (v_mfma_f64_16x16x4 for FP64, v_mfma_f32_16x16x4 for FP32).
 //
-// The launch configuration of a plan -- product form, tile-shape policy and
-// persistent grid size -- is chosen by autotune(): candidates are timed with
+// The launch configuration of a plan -- product form, tile-shape policy, K chunk,
+// persistent grid size and, for a small plan, its one-launch kernel -- is chosen
+// by autotune(): candidates are timed with
 // HIP events on the plan's own operands and the winner is cached under a
 // signature of the plan's block-size histogram, so a later plan with the
 // same histogram (the next iDMRG step at the same chi) reuses it.
