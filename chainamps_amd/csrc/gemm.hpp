@@ -13,10 +13,10 @@
 //
 // The launch configuration of a plan -- product form, tile-shape policy, K chunk,
 // persistent grid size and, for a small plan, its one-launch kernel -- is chosen
-// by autotune(): candidates are timed with
-// HIP events on the plan's own operands and the winner is cached under a
-// signature of the plan's block-size histogram, so a later plan with the
-// same histogram (the next iDMRG step at the same chi) reuses it.
+// by autotune(): candidates are timed with HIP events on the plan's own operands
+// and the winner is cached under a signature of the plan's block-size histogram,
+// so a later plan with the same histogram (the next iDMRG step at the same chi)
+// reuses it.
 #pragma once
 #include <cstdint>
 #include <vector>
