@@ -22,6 +22,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <type_traits>
@@ -1054,6 +1055,16 @@ void GemmPlan::build_rows(const std::vector<int>& eligible) {
   for (const Pass& q : passes) total += int64_t(probs[q.probs[0]].M) * probs[q.probs[0]].batch;
   int per = 1024;
   while (per > 16 * kRowWaves && total / per < 2048) per /= 2;
+  size_t nins = 0, nouts = 0, nblks = 0;
+  for (const Pass& q : passes) {
+    const GemmProb& p0 = probs[q.probs[0]];
+    for (int j = 0; j < p0.nseg; ++j) nins += static_cast<size_t>(segs[p0.seg0 + j].K);
+    nouts += static_cast<size_t>(q.nout);
+    nblks += q.probs.size() * static_cast<size_t>(p0.nseg);
+  }
+  row_in.reserve(nins);
+  row_out.reserve(nouts);
+  row_blk.reserve(nblks);
   std::vector<RowItem> first(passes.size());     // a pass's tables, without rows
   for (size_t qi = 0; qi < passes.size(); ++qi) {
     const Pass& q = passes[qi];
@@ -1202,19 +1213,23 @@ void GemmPlan::upload(hipStream_t s) {
     rows_uploaded = direct_uploaded = false;
     for (int m = 0; m < kTileModes; ++m) tiles_uploaded[m] = false;
   }
-  std::vector<char> host;
-  host.reserve(probs.size() * sizeof(GemmProb) + segs.size() * sizeof(GemmSeg) + rows.size() * sizeof(RowItem) +
-               (row_in.size() + row_out.size()) * sizeof(RowIn) + row_blk.size() * sizeof(RowBlk) + 1024);
-  std::vector<std::function<void(const char*)>> placed;
+  // (each byte of the staging copy is touched once: on the host a plan of many
+  // small blocks costs mostly the first use of its pages)
+  struct Placed {
+    const void* from;
+    size_t at, bytes;
+    std::function<void(const char*)> set;
+  };
+  size_t total = 0;
+  std::vector<Placed> placed;
   auto put = [&](const auto& v, auto& d) {
     d = nullptr;
     if (v.empty()) return;
-    const size_t at = (host.size() + 15) / 16 * 16;
-    host.resize(at + v.size() * sizeof(v[0]));
-    std::memcpy(host.data() + at, v.data(), v.size() * sizeof(v[0]));
-    placed.emplace_back([&d, at](const char* base) {
-      d = reinterpret_cast<std::remove_reference_t<decltype(d)>>(base + at);
-    });
+    const size_t at = (total + 15) / 16 * 16;
+    total = at + v.size() * sizeof(v[0]);
+    placed.push_back(Placed{v.data(), at, v.size() * sizeof(v[0]), [&d, at](const char* base) {
+                              d = reinterpret_cast<std::remove_reference_t<decltype(d)>>(base + at);
+                            }});
   };
   if (!uploaded) {
     put(probs, d_probs);
@@ -1230,10 +1245,14 @@ void GemmPlan::upload(hipStream_t s) {
   for (int m = 0; m < kTileModes; ++m)
     if (built[m] && !tiles_uploaded[m])
       for (int t = 0; t < kNumTileShapes; ++t) put(tiles[m][t], d_tiles[m][t]);
-  if (!host.empty()) {
-    DevBuf<char> buf(host.size());
-    buf.upload(host.data(), host.size(), s);
-    for (auto& set : placed) set(buf.get());
+  if (total) {
+    DevBuf<char> buf(total);
+    const std::unique_ptr<char[]> host(new char[total]);
+    for (const Placed& p : placed) {
+      std::memcpy(host.get() + p.at, p.from, p.bytes);
+      p.set(buf.get());
+    }
+    buf.upload(host.get(), total, s);
     d_bufs.push_back(std::move(buf));
   }
   uploaded = direct_uploaded = rows_uploaded = true;
